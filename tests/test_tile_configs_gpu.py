@@ -1,0 +1,93 @@
+"""The layer GEMMs choose their tile by the number of rows. Every output takes its K blocks in the same order whatever
+the tile, so a row's result must not depend on it: each kernel over `rows` rows, on both sides of every limit of the
+rules, against the same rows taken in pieces of at most 1025 (which run the smallest tiles, and which the parity tests
+check against the oracle), bit for bit."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+T, D, HIDP, PXH = 1025, 1024, 2816, 4736
+F32, U8 = torch.float32, torch.uint8
+
+
+def _codes(g, dev, *shape):
+    return torch.randn(*shape, generator=g, device=dev).to(torch.float8_e4m3fn).view(U8)
+
+
+class _W:
+    """random weight codes [N][K] and block scales, or pack24 values and indices"""
+
+    def __init__(self, g, dev, N, K, sp):
+        self.s = torch.rand(N // 128, K // 128, generator=g, device=dev) * 0.01
+        self.v = _codes(g, dev, N // 16, K // 128, 64, 16) if sp else _codes(g, dev, N, K)
+        # index nibbles p0 | p1 << 2 with p0 < p1: 0x4 (0, 1), 0xe (2, 3), 0x9 (1, 2)
+        self.x = torch.tensor([0x4E944E94, 0x4E9494E4, 0x44444444, -0x11111112], dtype=torch.int32, device=dev)
+        self.x = self.x[torch.randint(0, 4, (N // 16, K // 128, 64), generator=g, device=dev)].contiguous() if sp else None
+
+    def args(self, X):
+        return (X.ptr(self.v),) + ((X.ptr(self.x),) if self.x is not None else ()) + (X.ptr(self.s),)
+
+
+def _pieces(rows):
+    return [(r, min(r + T, rows)) for r in range(0, rows, T)]
+
+
+@pytest.mark.parametrize("sparse", [False, True])
+@pytest.mark.parametrize("rows", [1, 65, 1408, 1409, 4096, 4097, 8192, 8200, 16400])
+def test_rows_do_not_depend_on_the_tile(dev, xt, rows, sparse):
+    print(f"tile configurations: {rows} rows, sparse {sparse}", flush=True)
+    L, P, st = xt.lib, xt.ptr, torch.cuda.current_stream().cuda_stream
+    sfx = "_sp" if sparse else ""
+    g = torch.Generator(device=dev)
+    g.manual_seed(rows)
+    lds = rows + 256             # a piece's last tile reads scales (of rows it drops) up to 127 rows past its own
+    h8, hs = _codes(g, dev, rows, D), torch.rand(8, lds, generator=g, device=dev) * 0.01
+    m8, ms = _codes(g, dev, rows, HIDP), torch.rand(22, lds, generator=g, device=dev) * 0.01
+    stat = torch.rand(22, lds, 2, generator=g, device=dev) * 20
+    x0 = torch.randn(rows, D, generator=g, device=dev).half()
+    cn, dn = torch.rand(D, generator=g, device=dev), torch.rand(D, generator=g, device=dev)
+    wo, w1, w2 = (_W(g, dev, *s, sparse) for s in ((D, D), (2 * HIDP, D), (D, HIDP)))
+
+    def run(bounds):
+        xo, xf = x0.clone(), x0.clone()
+        mo, so, to = (torch.zeros(rows, HIDP, dtype=U8, device=dev), torch.zeros(22, lds, device=dev),
+                      torch.zeros(22, lds, 2, device=dev))
+        for a, b in bounds:
+            n = b - a
+            at = lambda t: P(t.reshape(-1)[a * t.stride(0):])           # row a of [rows][..]
+            pl = lambda t: P(t.reshape(-1)[a * t.stride(1):])           # row a of every scale plane
+            assert getattr(L, "eva_k_oproj" + sfx)(at(h8), pl(hs), lds, *wo.args(xt), at(xo), n, st) == 0
+            assert getattr(L, "eva_k_fc1" + sfx)(at(h8), pl(hs), lds, *w1.args(xt), at(mo), pl(so), pl(to), n, st) == 0
+            assert getattr(L, "eva_k_fc2" + sfx)(at(m8), pl(ms), lds, *w2.args(xt), pl(stat), P(cn), P(dn), at(xf), n, st) == 0
+        torch.cuda.synchronize()
+        return xo, xf, mo, so, to
+
+    for got, ref in zip(run([(0, rows)]), run(_pieces(rows))):
+        assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("sparse", [False, True])
+@pytest.mark.parametrize("nb", [2, 3, 6, 7])
+def test_qkv_rows_do_not_depend_on_the_tile(dev, xt, nb, sparse):
+    print(f"qkv tile configurations: {nb} images, sparse {sparse}", flush=True)
+    L, P, st = xt.lib, xt.ptr, torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=dev)
+    g.manual_seed(nb)
+    rows = nb * T
+    lds = rows + 256
+    h8, hs = _codes(g, dev, rows, D), torch.rand(8, lds, generator=g, device=dev) * 0.01
+    cs = torch.rand(1024, 32, 2, generator=g, device=dev)
+    w = _W(g, dev, 3 * D, D, sparse)
+
+    def run(step):
+        q, k, v = (torch.zeros(nb, 16, 1088 * 64, dtype=torch.int16, device=dev) for _ in range(3))
+        for b in range(0, nb, step):
+            at = lambda t: P(t[b:])
+            assert getattr(L, "eva_k_qkv" + ("_sp" if sparse else ""))(
+                P(h8[b * T:]), P(hs.reshape(-1)[b * T:]), lds, *w.args(xt), P(cs), at(q), at(k), at(v), step * T, st) == 0
+        torch.cuda.synchronize()
+        return q, k, v
+
+    for got, ref in zip(run(nb), run(1)):
+        assert torch.equal(got, ref)

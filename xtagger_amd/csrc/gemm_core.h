@@ -47,7 +47,8 @@ struct BsCfg {
     static constexpr int A_BYTES = BM * 128;
     static constexpr int B_BYTES = BN * 128;
     static constexpr int S_BYTES = BM * 4;     // activation scales of the BM rows
-    static constexpr int SW_BYTES = 256;       // weight scales of the BN / 128 column blocks (one 64-lane dword load)
+    static constexpr int SW_BYTES = 256;       // weight scales of the NB column blocks (one 64-lane dword load)
+    static constexpr int NB = (BN + 127) / 128;  // 128-column weight blocks of the tile (a 64-column tile sits in one)
     static constexpr int STAGE = A_BYTES + B_BYTES + S_BYTES + SW_BYTES;
     static constexpr int LDS = NS * STAGE;
     static constexpr int LA = BM / (8 * NW);  // 1 KB A loads (8 rows) per wave per stage
@@ -58,7 +59,7 @@ struct BsCfg {
     static_assert(WN <= 128 && 128 % WN == 0, "a wave's columns must sit in one weight block");
     static_assert(LA * 8 * NW == BM && LB * 8 * NW == BN, "tile rows must split evenly over the waves");
     static_assert(BM % 64 == 0 && SL < NW, "scale loads: one wave per 64 rows plus one for the weight scales");
-    static_assert(BN / 128 <= 64, "weight-scale load covers at most 64 column blocks");
+    static_assert(NB <= 64 && (BN % 128 == 0 || 128 % BN == 0), "whole weight blocks, or a tile inside one");
     static_assert(NS >= 2 && LDS <= 160 * 1024, "the stages must fit the 160 KB LDS");
     // 2:4-sparse weights (bs_mainloop_sp): per stage BN / 16 compressed 1 KB value blocks and 256-byte index blocks
     static constexpr int LV = BN / (16 * NW);   // value (and index) blocks per wave per stage
@@ -104,6 +105,14 @@ __device__ __forceinline__ void wait_vmem_n()
 {
     static_assert(N >= 0 && N < 64, "vmcnt range");
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// wait until all but the min(S, later) newest groups of L loads have landed (later: wave-uniform)
+template <int S, int L>
+__device__ __forceinline__ void wait_stages(int later)
+{
+    if constexpr (S == 0) wait_vmem();
+    else if (later >= S) wait_vmem_n<S * L>();
+    else wait_stages<S - 1, L>(later);
 }
 // block barrier after this wave's LDS reads have returned; no fence (the LDS DMA waits are explicit)
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
@@ -161,7 +170,7 @@ struct BsOperands {
         } else {                    // weight scales of column blocks n0 / 128 + lane (the last waves repeat it)
             const int nbt = Npad >> 7, nb = (n0 >> 7) + lane;
             rs = buf_desc(sw, (uint32_t)nbt * (uint32_t)KB * 4u);
-            s_off = (lane < C::BN / 128 && nb < nbt) ? (uint32_t)(nb * KB) * 4u : XT_OOR;
+            s_off = (lane < C::NB && nb < nbt) ? (uint32_t)(nb * KB) * 4u : XT_OOR;
             s_step = 4u;
             m0_s = (uint32_t)(C::A_BYTES + C::B_BYTES + C::S_BYTES);
         }
@@ -238,6 +247,10 @@ __device__ __forceinline__ void bs_step(const uint8_t *st, int wm0, int wn0, v4f
     }
 }
 
+// Wave tiles that the fixed-order step serves
+template <class C>
+constexpr bool BsFixed = (C::TM == 4 || C::TM == 2) && (C::TN == 8 || C::TN == 4 || C::TN == 2);
+
 // The same K step for 64 x 128 and 64 x 64 wave tiles (TM = 4, TN = 8 or 4) in a fixed issue order (for 64 x 64, the
 // single GEMM's 128 x 128 tiles, 12% faster than bs_step at M = 1025). The matrix-core instructions and
 // the promotion fmas are single-instruction asm statements, and every LDS read sits between them, so the compiler
@@ -261,22 +274,21 @@ __device__ __forceinline__ void fmac_asm(float &acc, float p, float s)
     asm volatile("v_fmac_f32 %0, %1, %2" : "+v"(acc) : "v"(p), "v"(s) : "memory");
 }
 
-// Promotion of a step's last three MFMAs (row tiles 1-3 of the last column tile, ring slots 1-3) with that step's
-// scales scp
+// Promotion of a step's last three MFMAs (ring slots t & 3) with that step's scales scp
 template <class C, bool TR = false>
 __device__ __forceinline__ void bs_step_fixed_flush(v4f (&acc)[C::TM][C::TN], const v4f (&pr)[4],
                                                     const float (&scp)[3][4])
 {
-    constexpr int J = C::TN - 1;
 #pragma unroll
     for (int q = 0; q < 3; q++) {
-        const v4f p = pr[1 + q];
-        float x0 = acc[1 + q][J][0], x1 = acc[1 + q][J][1], x2 = acc[1 + q][J][2], x3 = acc[1 + q][J][3];
+        const int u = C::TM * C::TN - 3 + q, ju = u / C::TM, iu = u % C::TM;
+        const v4f p = pr[u & 3];
+        float x0 = acc[iu][ju][0], x1 = acc[iu][ju][1], x2 = acc[iu][ju][2], x3 = acc[iu][ju][3];
         fmac_asm(x0, p[0], scp[q][0]);
         fmac_asm(x1, p[1], scp[q][TR ? 0 : 1]);
         fmac_asm(x2, p[2], scp[q][TR ? 0 : 2]);
         fmac_asm(x3, p[3], scp[q][TR ? 0 : 3]);
-        acc[1 + q][J] = v4f{x0, x1, x2, x3};
+        acc[iu][ju] = v4f{x0, x1, x2, x3};
     }
 }
 
@@ -285,33 +297,31 @@ __device__ __forceinline__ void bs_step_fixed(const uint8_t *st, int wm0, int wn
                                               const BsOperands<C> &op, uint32_t dstage, int dkb, v4f (&pr)[4],
                                               float (&scp)[3][4], bool carry)
 {
-    static_assert(C::TM == 4 && (C::TN == 8 || C::TN == 4) && C::LPS < 4 * C::TN,
-                  "schedule written for 64 x 128 and 64 x 64 wave tiles");
-    constexpr int LAG = 3, NM = 4 * C::TN;
+    static_assert(BsFixed<C>, "wave tiles of 4 or 2 row tiles");
+    constexpr int LAG = 3, NM = C::TM * C::TN, PER = (C::LPS + NM - 2) / (NM - 1);  // loads after each MFMA from 1 on
     const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
     const uint8_t *ta = st, *tb = st + C::A_BYTES;
     const float *ts = (const float *)(st + C::A_BYTES + C::B_BYTES);
-    v8i a[4], b[3];
+    v8i a[C::TM], b[3];
     b[0] = ld_frag(tb, wn0);
     a[0] = ld_frag(ta, wm0);
     asm volatile("" ::: "memory");  // the first MFMA waits for these four reads only
     if (carry) bs_step_fixed_flush<C, TR>(acc, pr, scp);  // the previous step's last three MFMAs, while the reads land
     const float swv = *(const float *)(st + C::A_BYTES + C::B_BYTES + C::S_BYTES + 4 * (wn0 >> 7));
-    float4 s4[4];
+    float4 s4[C::TM];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < C::TM; i++) {
         if constexpr (TR) s4[i].x = ts[wm0 + 16 * i + c16];  // TR: one row per lane and row tile
         else s4[i] = *(const float4 *)(ts + wm0 + 16 * i + 4 * g);
     }
     asm volatile("" ::: "memory");
-    a[1] = ld_frag(ta, wm0 + 16);
-    a[2] = ld_frag(ta, wm0 + 32);
-    a[3] = ld_frag(ta, wm0 + 48);
+#pragma unroll
+    for (int i = 1; i < C::TM; i++) a[i] = ld_frag(ta, wm0 + 16 * i);
     b[1] = ld_frag(tb, wn0 + 16);
     asm volatile("" ::: "memory");
-    float sc[4][4];
+    float sc[C::TM][4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < C::TM; i++) {
         if constexpr (TR) {
             sc[i][0] = s4[i].x * swv;
         } else {
@@ -320,14 +330,18 @@ __device__ __forceinline__ void bs_step_fixed(const uint8_t *st, int wm0, int wn
     }
 #pragma unroll
     for (int t = 0; t < NM; t++) {
-        const int j = t >> 2, i = t & 3;
+        const int j = t / C::TM, i = t % C::TM;
         if constexpr (TR) mfma_asm(pr[t % (LAG + 1)], b[j % 3], a[i]);  // the tile transposed: weights as A
         else mfma_asm(pr[t % (LAG + 1)], a[i], b[j % 3]);
         if (i == 0 && j + 2 < C::TN) b[(j + 2) % 3] = ld_frag(tb, wn0 + 16 * (j + 2));
-        if (t >= 1 && t <= C::LPS && dkb >= 0) op.issue_one(t - 1, dstage, dkb);
+        if (t >= 1 && (t - 1) * PER < C::LPS && dkb >= 0) {
+#pragma unroll
+            for (int e = 0; e < PER; e++)
+                if ((t - 1) * PER + e < C::LPS) op.issue_one((t - 1) * PER + e, dstage, dkb);
+        }
         if (t == LAG) asm volatile("s_nop 7" ::: "memory");
         if (t >= LAG) {
-            const int u = t - LAG, ju = u >> 2, iu = u & 3;
+            const int u = t - LAG, ju = u / C::TM, iu = u % C::TM;
             const v4f p = pr[u % (LAG + 1)];
             float x0 = acc[iu][ju][0], x1 = acc[iu][ju][1], x2 = acc[iu][ju][2], x3 = acc[iu][ju][3];
             fmac_asm(x0, p[0], sc[iu][0]);
@@ -340,10 +354,10 @@ __device__ __forceinline__ void bs_step_fixed(const uint8_t *st, int wm0, int wn
 #pragma unroll
     for (int q = 0; q < 3; q++)
 #pragma unroll
-        for (int r = 0; r < (TR ? 1 : 4); r++) scp[q][r] = sc[1 + q][r];  // the last three MFMAs: row tiles 1-3
+        for (int r = 0; r < (TR ? 1 : 4); r++) scp[q][r] = sc[(NM - 3 + q) % C::TM][r];  // the last three MFMAs
 }
 
-// The K step of a wave of a partial last row tile whose rows below M fill only its first TMV < 4 row tiles of 16:
+// The K step of a wave of a partial last row tile whose rows below M fill only its first TMV < TM row tiles of 16:
 // those row tiles' MFMAs and promotions, with the operands, order of promotion and instructions bs_step_fixed uses
 // for them (so their accumulators are bit-identical), the others left at zero as the zero rows past M would leave
 // them. The stage's loads go out first, all at once.
@@ -351,8 +365,7 @@ template <class C, int TMV, bool TR = false>
 __device__ __forceinline__ void bs_step_rows(const uint8_t *st, int wm0, int wn0, v4f (&acc)[C::TM][C::TN],
                                              const BsOperands<C> &op, uint32_t dstage, int dkb)
 {
-    static_assert(C::TM == 4 && (C::TN == 8 || C::TN == 4) && TMV >= 1 && TMV < 4,
-                  "partial row tiles of 64 x 128 and 64 x 64 wave tiles");
+    static_assert(BsFixed<C> && TMV >= 1 && TMV < C::TM, "some but not all row tiles of the wave");
     constexpr int LAG = 3, NM = C::TN * TMV;
     if (dkb >= 0) op.issue(dstage, dkb);
     const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
@@ -457,17 +470,16 @@ __device__ __forceinline__ void bs_mainloop(const uint8_t *__restrict__ A, int l
         int cs = 0, is = C::NS - 1;  // stage computed now, stage issued now
         for (int kb = 0; kb < KB; kb++) {
             // stage kb must be resident; the min(NS - 2, KB - 1 - kb) stages issued after it may stay in flight
-            if (kb + C::NS - 2 < KB) wait_vmem_n<(C::NS - 2) * C::LPS>();
-            else wait_vmem();
+            wait_stages<C::NS - 2, C::LPS>(KB - 1 - kb);
             lds_barrier();  // every wave's part of stage kb landed; every wave finished reading stage kb - 1
             step(smem + cs * C::STAGE, base + is * C::STAGE, kb + C::NS - 1 < KB ? kb + C::NS - 1 : -1);
             cs = cs == C::NS - 1 ? 0 : cs + 1;
             is = is == C::NS - 1 ? 0 : is + 1;
         }
     };
-    if constexpr (C::TM == 4 && (C::TN == 8 || C::TN == 4)) {
-        if (live > 32) {
-            v4f pr[4];          // the MFMA result ring, and the scales of the last step's MFMAs 29-31 (their
+    if constexpr (BsFixed<C>) {
+        if (live > 8 * C::TM) {
+            v4f pr[4];          // the MFMA result ring, and the scales of the last step's last three MFMAs (their
             float scp[3][4];    // promotions run at the start of the next step)
             int kbi = 0;
             kloop([&](const uint8_t *st, uint32_t dst, int dkb) {
@@ -476,9 +488,9 @@ __device__ __forceinline__ void bs_mainloop(const uint8_t *__restrict__ A, int l
             });
             asm volatile("s_nop 7\n\ts_nop 7" ::: "memory");  // 12+ wait states after the last MFMA
             bs_step_fixed_flush<C, TR>(acc, pr, scp);
-        } else if (live > 16)
+        } else if (C::TM == 4 && live > 16)
             kloop([&](const uint8_t *st, uint32_t dst, int dkb) {
-                bs_step_rows<C, 2, TR>(st, wm0, wn0, acc, op, dst, dkb);
+                bs_step_rows<C, C::TM / 2, TR>(st, wm0, wn0, acc, op, dst, dkb);
             });
         else if (live > 0)
             kloop([&](const uint8_t *st, uint32_t dst, int dkb) {
@@ -548,7 +560,7 @@ struct BsSpOperands {
         } else {
             const int nbt = Npad >> 7, nb = (n0 >> 7) + lane;
             rs = buf_desc(sw, (uint32_t)nbt * (uint32_t)KB * 4u);
-            s_off = (lane < C::BN / 128 && nb < nbt) ? (uint32_t)(nb * KB) * 4u : XT_OOR;
+            s_off = (lane < C::NB && nb < nbt) ? (uint32_t)(nb * KB) * 4u : XT_OOR;
             s_step = 4u;
             m0_s = (uint32_t)(C::A_BYTES + C::V_BYTES + C::X_BYTES + C::S_BYTES);
         }
@@ -601,51 +613,54 @@ template <class C>
 __device__ __forceinline__ void bs_step_sp(const uint8_t *st, int wm0, int wn0, v4f (&accT)[C::TN][C::TM],
                                            const BsSpOperands<C> &op, uint32_t dstage, int dkb, uint32_t zl)
 {
-    static_assert(C::TM == 4 && C::TN >= 2 && C::LPS_SP < C::TN * C::TM, "schedule written for 64-row wave tiles");
+    static_assert(BsFixed<C>, "wave tiles of 4 or 2 row tiles");
     const int lane = threadIdx.x & 63, c16 = lane & 15;
     const uint8_t *ta = st, *tv = st + C::A_BYTES, *tx = st + C::A_BYTES + C::V_BYTES;
     const float *ts = (const float *)(st + C::A_BYTES + C::V_BYTES + C::X_BYTES);
     // the wave's weight tiles j = 0 .. TN - 1 at tvl + 1024 j and txl + 256 j (constant offsets of one base each)
     const uint8_t *tvl = tv + (wn0 >> 4) * 1024 + 16 * lane, *txl = tx + (wn0 >> 4) * 256 + 4 * lane;
-    constexpr int NS = C::TN * C::TM, LAG = 3, R = 6;
+    constexpr int NS = C::TN * C::TM, LAG = 3, R = NS < 6 ? NS : 6, PER = (C::LPS_SP + NS - 2) / (NS - 1);
     v4i v[3];
     int x[3];
-    v8i xa[4];
+    v8i xa[C::TM];
     v[0] = *(const v4i *)tvl;
     x[0] = *(const int *)txl;
     xa[0] = ld_frag(ta, wm0);
     asm volatile("" ::: "memory");  // the first MFMA waits for these reads only
     const float swv = *(const float *)(st + C::A_BYTES + C::V_BYTES + C::X_BYTES + C::S_BYTES + 4 * (wn0 >> 7));
-    float sr[4];
+    float sr[C::TM];
 #pragma unroll
-    for (int i = 0; i < 4; i++) sr[i] = ts[wm0 + 16 * i + c16];
+    for (int i = 0; i < C::TM; i++) sr[i] = ts[wm0 + 16 * i + c16];
     asm volatile("" ::: "memory");
-    xa[1] = ld_frag(ta, wm0 + 16);
-    xa[2] = ld_frag(ta, wm0 + 32);
-    xa[3] = ld_frag(ta, wm0 + 48);
+#pragma unroll
+    for (int i = 1; i < C::TM; i++) xa[i] = ld_frag(ta, wm0 + 16 * i);
     v[1] = *(const v4i *)(tvl + 1024);
     x[1] = *(const int *)(txl + 256);
     asm volatile("" ::: "memory");
-    float sc[4];
+    float sc[C::TM];
 #pragma unroll
-    for (int i = 0; i < 4; i++) sc[i] = sr[i] * swv;
+    for (int i = 0; i < C::TM; i++) sc[i] = sr[i] * swv;
     v4f pr[R];
 #pragma unroll
     for (int r = 0; r < R; r++) lds_zero(pr[r], zl);
 #pragma unroll
     for (int t = 0; t < NS + LAG; t++) {
         if (t < NS) {
-            const int j = t >> 2, i = t & 3;
+            const int j = t / C::TM, i = t % C::TM;
             smfmac_asm(pr[t % R], v[j % 3], xa[i], x[j % 3]);
             if (i == 0 && j + 2 < C::TN) {
                 v[(j + 2) % 3] = *(const v4i *)(tvl + 1024 * (j + 2));
                 x[(j + 2) % 3] = *(const int *)(txl + 256 * (j + 2));
             }
-            if (t >= 1 && t <= C::LPS_SP && dkb >= 0) op.issue_one(t - 1, dstage, dkb);
+            if (t >= 1 && (t - 1) * PER < C::LPS_SP && dkb >= 0) {
+#pragma unroll
+                for (int e = 0; e < PER; e++)
+                    if ((t - 1) * PER + e < C::LPS_SP) op.issue_one((t - 1) * PER + e, dstage, dkb);
+            }
         }
         if (t == LAG) asm volatile("s_nop 7" ::: "memory");
         if (t >= LAG) {
-            const int u = t - LAG, ju = u >> 2, iu = u & 3;
+            const int u = t - LAG, ju = u / C::TM, iu = u % C::TM;
             const v4f p = pr[u % R];
             float x0 = accT[ju][iu][0], x1 = accT[ju][iu][1], x2 = accT[ju][iu][2], x3 = accT[ju][iu][3];
             fmac_asm(x0, p[0], sc[iu]);
@@ -659,13 +674,13 @@ __device__ __forceinline__ void bs_step_sp(const uint8_t *st, int wm0, int wn0, 
 }
 
 // The transposed wave tile (accT[n tile][m tile][r]: n = wn0 + 16 i + 4 (lane >> 4) + r, m = wm0 + 16 j + (lane & 15))
-// to the dense accumulator layout of bs_mainloop, through the wave's own 64 x 68 fp32 slice of shared memory
-// (slices at `slices` + wave * 17408 bytes), 64 columns per pass.
+// to the dense accumulator layout of bs_mainloop, through the wave's own WM x 68 fp32 slice of shared memory
+// (17408 bytes for 64 rows), 64 columns per pass.
 template <class C>
 __device__ __forceinline__ void bs_sp_to_dense(uint8_t *slices, v4f (&accT)[C::TN][C::TM], v4f (&acc)[C::TM][C::TN])
 {
-    static_assert(C::TM == 4 && C::TN % 4 == 0, "64-row wave tiles, whole 64-column passes");
-    float *tr = (float *)(slices + (threadIdx.x >> 6) * (64 * 68 * 4));
+    static_assert(C::TN % 4 == 0, "whole 64-column passes");
+    float *tr = (float *)(slices + (threadIdx.x >> 6) * (C::WM * 68 * 4));
     const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
 #pragma unroll
     for (int pass = 0; pass < C::TN / 4; pass++) {
@@ -673,13 +688,13 @@ __device__ __forceinline__ void bs_sp_to_dense(uint8_t *slices, v4f (&accT)[C::T
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
-            for (int j = 0; j < 4; j++)
+            for (int j = 0; j < C::TM; j++)
                 *(float4 *)(tr + (16 * j + c16) * 68 + 16 * i + 4 * g) =
                     make_float4(accT[4 * pass + i][j][0], accT[4 * pass + i][j][1], accT[4 * pass + i][j][2],
                                 accT[4 * pass + i][j][3]);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slice is the wave's own: no block barrier needed
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+        for (int i = 0; i < C::TM; i++)
 #pragma unroll
             for (int j = 0; j < 4; j++)
 #pragma unroll
@@ -726,8 +741,7 @@ __device__ __forceinline__ void bs_mainloop_sp_t(const uint8_t *__restrict__ A, 
                       __builtin_amdgcn_readfirstlane(n0 + wn0) < (Nlive < 0 ? Npad : Nlive);
     int cs = 0, is = C::NS - 1;
     for (int kb = 0; kb < KB; kb++) {
-        if (kb + C::NS - 2 < KB) wait_vmem_n<(C::NS - 2) * C::LPS_SP>();
-        else wait_vmem();
+        wait_stages<C::NS - 2, C::LPS_SP>(KB - 1 - kb);
         lds_barrier();
         const int dkb = kb + C::NS - 1 < KB ? kb + C::NS - 1 : -1;
         if constexpr (SPREAD) {

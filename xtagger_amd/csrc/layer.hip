@@ -15,16 +15,16 @@
 // i = lane & 15, so a lane holds dims 4i .. 4i + 3, the rotary pairs 2i and 2i + 1 whole: their (cos, sin) come in one
 // 16-byte load and the rotated dims leave in one 8-byte store. q rows carry log2(e)/8 (export_eva.py:71).
 // ---------------------------------------------------------------------------------------------------------------
-template <bool SP>
-__global__ void __launch_bounds__(LayerCfg::NT) k_qkv(const uint8_t *__restrict__ h8, const float *__restrict__ hs,
+template <class C, bool SP>
+__global__ void __launch_bounds__(C::NT) k_qkv(const uint8_t *__restrict__ h8, const float *__restrict__ hs,
                                                      int lds, const uint8_t *__restrict__ w,
                                                      const uint32_t *__restrict__ wx,
                                                      const float *__restrict__ ws, const float *__restrict__ cs,
                                                      uint16_t *__restrict__ q, uint16_t *__restrict__ k,
                                                      uint16_t *__restrict__ vt, int rows)
 {
-    using C = LayerCfg;
-    __shared__ __attribute__((aligned(16))) uint8_t smem[LAYER_SMEM];
+    constexpr int NH = C::TN / 4, TRLD = LayerMem<C>::TRLD;  // heads per wave
+    __shared__ __attribute__((aligned(16))) uint8_t smem[LayerMem<C>::SMEM];
     v4f acc[C::TM][C::TN];
     int m0, n0, wm0, wn0;
     layer_tile<C>(rows, 3 * XT_D, m0, n0);
@@ -32,21 +32,22 @@ __global__ void __launch_bounds__(LayerCfg::NT) k_qkv(const uint8_t *__restrict_
     bs_wave_origin<C>(wm0, wn0);
     const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
     const int part = n0 >> 10, head0 = ((n0 & 1023) + wn0) >> 6;
-    // v: the wave's 64 rows x 128 dims (two heads) are transposed through its own LDS slice ([128 dims][68] bf16,
-    // padded rows), then lanes walk rows (consecutive tokens). The slice takes the tile in whichever layout the main
+    // v: the wave's rows x dims (one or two heads) are transposed through its own LDS slice ([WN dims][WM + 4] bf16,
+    // padded rows), then lanes walk rows (consecutive tokens; two dims at a time where the wave has 32 rows). The slice takes the tile in whichever layout the main
     // loop leaves it: the sparse loop's transposed tile directly (no pass through the dense layout first), the dense
     // tile as one 8-byte write of four consecutive tokens per (row tile, column tile).
-    uint16_t *tr = (uint16_t *)(smem + (threadIdx.x >> 6) * 128 * 68 * 2);
+    uint16_t *tr = (uint16_t *)(smem + (threadIdx.x >> 6) * LayerMem<C>::TRSLICE);
     auto v_out = [&]() {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        const int m = m0 + wm0 + lane;
+        constexpr int DS = 64 / C::WM;  // dims per store instruction
+        const int row = lane % C::WM, d0 = lane / C::WM, m = m0 + wm0 + row;
         if (m < rows) {
             const int b = m / XT_T, t = m - b * XT_T;
 #pragma unroll
-            for (int hh = 0; hh < 2; hh++) {
+            for (int hh = 0; hh < NH; hh++) {
                 uint16_t *dst = vt + ((size_t)b * XT_NH + head0 + hh) * XT_HD * XT_TP + t;
 #pragma unroll 8
-                for (int d = 0; d < XT_HD; d++) dst[(size_t)d * XT_TP] = tr[(64 * hh + d) * 68 + lane];
+                for (int d = d0; d < XT_HD; d += DS) dst[(size_t)d * XT_TP] = tr[(64 * hh + d) * TRLD + row];
             }
         }
     };
@@ -60,7 +61,7 @@ __global__ void __launch_bounds__(LayerCfg::NT) k_qkv(const uint8_t *__restrict_
                 for (int i = 0; i < C::TM; i++)
 #pragma unroll
                     for (int r = 0; r < 4; r++)
-                        tr[(16 * j + 4 * g + r) * 68 + 16 * i + c16] = (uint16_t)pk_bf16(accT[j][i][r], 0.f);
+                        tr[(16 * j + 4 * g + r) * TRLD + 16 * i + c16] = (uint16_t)pk_bf16(accT[j][i][r], 0.f);
             v_out();
             return;
         }
@@ -92,7 +93,7 @@ __global__ void __launch_bounds__(LayerCfg::NT) k_qkv(const uint8_t *__restrict_
             for (int r = 0; r < 4; r++) {
                 const int b = img[i][r], t = tok[i][r];
 #pragma unroll
-                for (int hh = 0; hh < 2; hh++) {
+                for (int hh = 0; hh < NH; hh++) {
                     uint32_t two[2];
 #pragma unroll
                     for (int p = 0; p < 2; p++) {
@@ -118,7 +119,7 @@ __global__ void __launch_bounds__(LayerCfg::NT) k_qkv(const uint8_t *__restrict_
 #pragma unroll
         for (int j = 0; j < C::TN; j++) {
             typedef unsigned v2u __attribute__((ext_vector_type(2)));
-            *(v2u *)(tr + (16 * j + c16) * 68 + 16 * i + 4 * g) =
+            *(v2u *)(tr + (16 * j + c16) * TRLD + 16 * i + 4 * g) =
                 v2u{pk_bf16(acc[i][j][0], acc[i][j][1]), pk_bf16(acc[i][j][2], acc[i][j][3])};
         }
     v_out();
@@ -127,21 +128,19 @@ __global__ void __launch_bounds__(LayerCfg::NT) k_qkv(const uint8_t *__restrict_
 // ---------------------------------------------------------------------------------------------------------------
 // k_oproj: x [rows][1024] = f16(x + attn_out . Wo^T) (eva_kernels.cu:150-160, alpha folded into the block scales)
 // ---------------------------------------------------------------------------------------------------------------
-template <bool SP>
-__global__ void __launch_bounds__(LayerCfg::NT) k_oproj(const uint8_t *__restrict__ a8, const float *__restrict__ as,
+template <class C, bool SP>
+__global__ void __launch_bounds__(C::NT) k_oproj(const uint8_t *__restrict__ a8, const float *__restrict__ as,
                                                        int lds, const uint8_t *__restrict__ w,
                                                        const uint32_t *__restrict__ wx,
                                                        const float *__restrict__ ws, uint16_t *__restrict__ x, int rows)
 {
-    using C = LayerCfg;
-    __shared__ __attribute__((aligned(16))) uint8_t smem[LAYER_SMEM];
+    __shared__ __attribute__((aligned(16))) uint8_t smem[LayerMem<C>::SMEM];
     v4f acc[C::TM][C::TN];
     int m0, n0, wm0, wn0;
     layer_tile<C>(rows, XT_D, m0, n0);
     args_resident(x, lds, rows);
     // the transposed tile (sparse: as the sparse main loop leaves it; dense: TR) goes straight into the residual update
     if constexpr (SP) {
-        static_assert(C::LDS_SP <= LAYER_ROWSTAT, "sparse stages end before the row statistics");
         v4f accT[C::TN][C::TM];
         bs_mainloop_sp_t<C>(a8, XT_D, as, lds, w, wx, ws, rows, XT_D, XT_D, m0, n0, smem, accT);
         bs_wave_origin<C>(wm0, wn0);
@@ -163,18 +162,17 @@ __global__ void __launch_bounds__(LayerCfg::NT) k_oproj(const uint8_t *__restric
 // and the sums.
 // Each (row, block) partial has one writer: no atomics, deterministic.
 // ---------------------------------------------------------------------------------------------------------------
-template <bool SP, bool RS>
-__global__ void __launch_bounds__(LayerCfg::NT) k_fc1(const uint8_t *__restrict__ h8, const float *__restrict__ hs,
+template <class C, bool SP, bool RS>
+__global__ void __launch_bounds__(C::NT) k_fc1(const uint8_t *__restrict__ h8, const float *__restrict__ hs,
                                                      int lds, const uint8_t *__restrict__ w,
                                                      const uint32_t *__restrict__ wx,
                                                      const float *__restrict__ ws, uint8_t *__restrict__ m8,
                                                      float *__restrict__ ms, float *__restrict__ stat,
                                                      const float *__restrict__ rs, int rows)
 {
-    using C = LayerCfg;
     constexpr int NP = C::TN / 2;                        // SwiGLU tile pairs per wave (16 units each)
-    __shared__ __attribute__((aligned(16))) uint8_t smem[LAYER_SMEM];
-    static_assert(C::BM * 8 % C::NT == 0, "packing items split evenly over the threads");
+    __shared__ __attribute__((aligned(16))) uint8_t smem[LayerMem<C>::SMEM];
+    static_assert(C::BN == 256 && C::BM * 8 % C::NT == 0, "packing items split evenly over the threads");
     int m0, n0, wm0, wn0;
     layer_tile<C>(rows, 2 * XT_HIDP, m0, n0);
     args_resident(m8, ms, stat, lds, rows);
@@ -183,23 +181,22 @@ __global__ void __launch_bounds__(LayerCfg::NT) k_fc1(const uint8_t *__restrict_
     constexpr int nlive = 2 * ((XT_HID + 15) / 16 * 16);
     // h tile [BM rows][128 units] fp32 in LDS, 16-byte chunk c of row r at chunk c ^ (r & 7)
     float *ht = (float *)smem;
-    static_assert(C::BM * 128 * 4 <= LAYER_SMEM, "fc1 staging fits");
-    static_assert(NP == 4, "two chunk pairs per 64-unit half");
+    static_assert(C::BM * 128 * 4 <= LayerMem<C>::SMEM, "fc1 staging fits");
+    static_assert(NP == 4 || NP == 2, "64 or 32 units per wave");
     const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
     const int ct = n0 >> 8;
     // silu(g) x, hardware reciprocal (1 ulp)
     auto swiglu = [](float gg, float xx) { return (gg * __builtin_amdgcn_rcpf(1.0f + __expf(-gg))) * xx; };
     // The transposed tile (sparse: as the sparse main loop leaves it; dense: TR): lane (g, c16) holds units
-    // 64 wn + 16 p + 4 g + r (r = 0..3) of row wm0 + 16 i + c16 for tile pair p (gate tile 2p, value tile 2p + 1: the
-    // same unit in the same register), so each (i, p) is one 16-byte chunk, 16 wn + 8 (p >> 1) + (4 (p & 1) + g), of a
+    // wn0 / 2 + 16 p + 4 g + r (r = 0..3) of row wm0 + 16 i + c16 for tile pair p (gate tile 2p, value tile 2p + 1: the
+    // same unit in the same register), so each (i, p) is one 16-byte chunk, wn0 / 8 + 8 (p >> 1) + (4 (p & 1) + g), of a
     // row with row & 7 = c16 & 7: at tb[p & 1] + 2048 i + 32 (p >> 1) words.
     auto stage_h = [&](auto pair) {
         bs_wave_origin<C>(wm0, wn0);
-        const int wn = wn0 / C::WN;
         uint32_t tb[2];
 #pragma unroll
         for (int ph = 0; ph < 2; ph++)
-            tb[ph] = (uint32_t)((wm0 + c16) * 128 + (16 * wn + ((4 * ph + g) ^ (c16 & 7))) * 4);
+            tb[ph] = (uint32_t)((wm0 + c16) * 128 + (wn0 / 8 + ((4 * ph + g) ^ (c16 & 7))) * 4);
 #pragma unroll
         for (int i = 0; i < C::TM; i++)
 #pragma unroll
@@ -211,7 +208,6 @@ __global__ void __launch_bounds__(LayerCfg::NT) k_fc1(const uint8_t *__restrict_
             }
     };
     if constexpr (SP) {
-        static_assert(C::LDS_SP <= LAYER_ROWSTAT, "sparse stages end before the row statistics");
         v4f accT[C::TN][C::TM];
         bs_mainloop_sp_t<C>(h8, XT_D, hs, lds, w, wx, ws, rows, 2 * XT_HIDP, XT_D, m0, n0, smem, accT, BsNoPre(),
                             nlive);
@@ -281,22 +277,21 @@ __global__ void __launch_bounds__(LayerCfg::NT) k_fc1(const uint8_t *__restrict_
 // W~, d = W2 beta), mean / rstd of the SwiGLU row over 2730 units from k_fc1's 22 partials summed in block order:
 // mean = S / 2730, var = max(Q / 2730 - mean^2, 0), rstd = 1 / sqrt(var + 1e-6) (eva_kernels.cu:300-333).
 // ---------------------------------------------------------------------------------------------------------------
-template <bool SP>
-__global__ void __launch_bounds__(LayerCfg::NT) k_fc2(const uint8_t *__restrict__ m8, const float *__restrict__ ms,
+template <class C, bool SP>
+__global__ void __launch_bounds__(C::NT) k_fc2(const uint8_t *__restrict__ m8, const float *__restrict__ ms,
                                                      int lds, const uint8_t *__restrict__ w,
                                                      const uint32_t *__restrict__ wx,
                                                      const float *__restrict__ ws, const float *__restrict__ stat,
                                                      const float *__restrict__ cn, const float *__restrict__ dn,
                                                      uint16_t *__restrict__ x, int rows)
 {
-    using C = LayerCfg;
-    __shared__ __attribute__((aligned(16))) uint8_t smem[LAYER_SMEM];
+    using S = LayerMem<C>;
+    __shared__ __attribute__((aligned(16))) uint8_t smem[S::SMEM];
     v4f acc[C::TM][C::TN];
     int m0, n0, wm0, wn0;
     layer_tile<C>(rows, XT_D, m0, n0);
-    float2 *rs = (float2 *)(smem + LAYER_ROWSTAT);         // [BM rows] (rstd, -mean * rstd)
-    float2 *cd = (float2 *)(smem + LAYER_ROWSTAT + 2048);  // [BN columns] (c, d)
-    static_assert(C::BM * 8 <= 2048 && C::BN * 8 <= 2048, "row statistics and column terms fit their 2 KB each");
+    float2 *rs = (float2 *)(smem + S::ROWSTAT);              // [BM rows] (rstd, -mean * rstd)
+    float2 *cd = (float2 *)(smem + S::ROWSTAT + 8 * C::BM);  // [BN columns] (c, d)
     auto rowstats = [&]() {
         if (threadIdx.x < C::BM) {
             const int m = m0 + threadIdx.x;
@@ -337,7 +332,6 @@ __global__ void __launch_bounds__(LayerCfg::NT) k_fc2(const uint8_t *__restrict_
         return v;
     };
     if constexpr (SP) {
-        static_assert(C::LDS_SP <= LAYER_ROWSTAT, "sparse stages end before the row statistics");
         v4f accT[C::TN][C::TM];
         bs_mainloop_sp_t<C>(m8, XT_HIDP, ms, lds, w, wx, ws, rows, XT_D, XT_HIDP, m0, n0, smem, accT, rowstats);
         bs_wave_origin<C>(wm0, wn0);
@@ -517,6 +511,28 @@ __global__ void __launch_bounds__(256) k_pe(const uint16_t *__restrict__ in, con
 // ---------------------------------------------------------------------------------------------------------------
 // C-ABI launchers
 // ---------------------------------------------------------------------------------------------------------------
+// qkv's tiles: 128 x 128 while one round of two blocks per CU holds them (rows <= 2688: 17.2 -> 8.4 us at 1025 rows,
+// 18.5 -> 12.7 at 2050), and where 256 x 256 tiles would run a second round less than a quarter full (6150 rows: 34.3
+// -> 30.0 us); 256 x 256 elsewhere (20.6 against 22.1 us at 4100, 34.8 against 38.8 at 8200).
+template <class F>
+static void with_qkv_cfg(int rows, F f)
+{
+    const unsigned big = layer_grid<LayerCfg>(rows, 3 * XT_D);
+    if (rows <= 2688 || (big > 256 && big <= 320)) f(LayerMid{});
+    else f(LayerCfg{});
+}
+
+// fc1's tiles (a block holds all 256 columns of a 128-unit scale block): 128 x 256, 16 waves of 32 x 64, while they
+// fit the 256 CUs at once (rows <= 1408: 16.6 -> 10.2 us at 1025 rows); beyond that 256 x 256 (18.0 against 19.2 us at
+// 2050 rows, 50.4 against 58.3 at 8200).
+typedef BsCfg<128, 256, 4, 4, 3> Fc1Mid;
+template <class F>
+static void with_fc1_cfg(int rows, F f)
+{
+    if (rows <= 1408) f(Fc1Mid{});
+    else f(LayerCfg{});
+}
+
 template <bool SP>
 static int qkv_launch(const char *what, const void *h8, const float *hs, int lds, const void *w, const void *wx,
                       const float *ws, const float *cs, void *q, void *k, void *vt, int rows, void *stream)
@@ -524,9 +540,12 @@ static int qkv_launch(const char *what, const void *h8, const float *hs, int lds
     if (layer_rows_ok(what, rows, lds)) return -1;
     if (rows % XT_T) return xt_fail(what, "rows must be nb * 1025");
     if (!XT_ALIGNED(h8) || !XT_ALIGNED(w) || (SP && !wx)) return xt_fail(what, "h8 and w must be 16-byte aligned");
-    hipLaunchKernelGGL(k_qkv<SP>, dim3(layer_grid(rows, 3 * XT_D, LayerCfg::BM, LayerCfg::BN)), dim3(LayerCfg::NT), 0,
-                       (hipStream_t)stream, (const uint8_t *)h8, hs, lds, (const uint8_t *)w, (const uint32_t *)wx, ws,
-                       cs, (uint16_t *)q, (uint16_t *)k, (uint16_t *)vt, rows);
+    with_qkv_cfg(rows, [&](auto c) {
+        using C = decltype(c);
+        hipLaunchKernelGGL((k_qkv<C, SP>), dim3(layer_grid<C>(rows, 3 * XT_D)), dim3(C::NT), 0, (hipStream_t)stream,
+                           (const uint8_t *)h8, hs, lds, (const uint8_t *)w, (const uint32_t *)wx, ws, cs,
+                           (uint16_t *)q, (uint16_t *)k, (uint16_t *)vt, rows);
+    });
     return xt_check(what);
 }
 
@@ -536,9 +555,12 @@ static int oproj_launch(const char *what, const void *a8, const float *as, int l
 {
     if (layer_rows_ok(what, rows, lds)) return -1;
     if (!XT_ALIGNED(a8) || !XT_ALIGNED(w) || (SP && !wx)) return xt_fail(what, "a8 and w must be 16-byte aligned");
-    hipLaunchKernelGGL(k_oproj<SP>, dim3(layer_grid(rows, XT_D, LayerCfg::BM, LayerCfg::BN)), dim3(LayerCfg::NT), 0,
-                       (hipStream_t)stream, (const uint8_t *)a8, as, lds, (const uint8_t *)w, (const uint32_t *)wx, ws,
-                       (uint16_t *)x, rows);
+    with_res_cfg(rows, XT_D, [&](auto c) {
+        using C = decltype(c);
+        hipLaunchKernelGGL((k_oproj<C, SP>), dim3(layer_grid<C>(rows, XT_D)), dim3(C::NT), 0, (hipStream_t)stream,
+                           (const uint8_t *)a8, as, lds, (const uint8_t *)w, (const uint32_t *)wx, ws, (uint16_t *)x,
+                           rows);
+    });
     return xt_check(what);
 }
 
@@ -549,13 +571,16 @@ static int fc1_launch(const char *what, const void *h8, const float *hs, int lds
     if (layer_rows_ok(what, rows, lds)) return -1;
     if (!XT_ALIGNED(h8) || !XT_ALIGNED(w) || !XT_ALIGNED(m8) || !XT_ALIGNED(rs) || (SP && !wx))
         return xt_fail(what, "h8, w, m8, rs must be 16-byte aligned");
-    const dim3 grid(layer_grid(rows, 2 * XT_HIDP, LayerCfg::BM, LayerCfg::BN));
-    if (rs)
-        hipLaunchKernelGGL((k_fc1<SP, true>), grid, dim3(LayerCfg::NT), 0, (hipStream_t)stream, (const uint8_t *)h8, hs,
-                           lds, (const uint8_t *)w, (const uint32_t *)wx, ws, (uint8_t *)m8, ms, stat, rs, rows);
-    else
-        hipLaunchKernelGGL((k_fc1<SP, false>), grid, dim3(LayerCfg::NT), 0, (hipStream_t)stream, (const uint8_t *)h8, hs,
-                           lds, (const uint8_t *)w, (const uint32_t *)wx, ws, (uint8_t *)m8, ms, stat, rs, rows);
+    with_fc1_cfg(rows, [&](auto c) {
+        using C = decltype(c);
+        const dim3 grid(layer_grid<C>(rows, 2 * XT_HIDP));
+        if (rs)
+            hipLaunchKernelGGL((k_fc1<C, SP, true>), grid, dim3(C::NT), 0, (hipStream_t)stream, (const uint8_t *)h8, hs,
+                               lds, (const uint8_t *)w, (const uint32_t *)wx, ws, (uint8_t *)m8, ms, stat, rs, rows);
+        else
+            hipLaunchKernelGGL((k_fc1<C, SP, false>), grid, dim3(C::NT), 0, (hipStream_t)stream, (const uint8_t *)h8,
+                               hs, lds, (const uint8_t *)w, (const uint32_t *)wx, ws, (uint8_t *)m8, ms, stat, rs, rows);
+    });
     return xt_check(what);
 }
 
@@ -566,9 +591,12 @@ static int fc2_launch(const char *what, const void *m8, const float *ms, int lds
 {
     if (layer_rows_ok(what, rows, lds)) return -1;
     if (!XT_ALIGNED(m8) || !XT_ALIGNED(w) || (SP && !wx)) return xt_fail(what, "m8 and w must be 16-byte aligned");
-    hipLaunchKernelGGL(k_fc2<SP>, dim3(layer_grid(rows, XT_D, LayerCfg::BM, LayerCfg::BN)), dim3(LayerCfg::NT), 0,
-                       (hipStream_t)stream, (const uint8_t *)m8, ms, lds, (const uint8_t *)w, (const uint32_t *)wx, ws,
-                       stat, cn, dn, (uint16_t *)x, rows);
+    with_res_cfg(rows, XT_HIDP, [&](auto c) {
+        using C = decltype(c);
+        hipLaunchKernelGGL((k_fc2<C, SP>), dim3(layer_grid<C>(rows, XT_D)), dim3(C::NT), 0, (hipStream_t)stream,
+                           (const uint8_t *)m8, ms, lds, (const uint8_t *)w, (const uint32_t *)wx, ws, stat, cn, dn,
+                           (uint16_t *)x, rows);
+    });
     return xt_check(what);
 }
 

@@ -6,16 +6,27 @@
 #include "xt_abi.h"
 
 typedef BsCfg<256, 256, 4, 2, 2> LayerCfg;  // 8 waves of 64 x 128: two heads (qkv) or 64 SwiGLU units (fc1) per wave
+// Smaller tiles for grids that LayerCfg would leave mostly idle (with_res_cfg, and qkv's and fc1's own rules). Every
+// output takes its K blocks in the same order whatever the tile, so the choice never changes a bit.
+typedef BsCfg<128, 128, 4, 2, 2> LayerMid;  // 8 waves of 32 x 64, two blocks per CU
+typedef BsCfg<64, 128, 2, 2, 3> LayerSml;   // 4 waves of 32 x 64, three stages, two blocks per CU
 
-// Shared memory of the layer kernels: the main-loop stages, reused by the epilogues (one 64 x 68 fp32 residual slice
-// per wave, one [128][68] bf16 transpose slice per wave, or the fc1 h tile), then 2 KB of per-row statistics and
-// 2 KB of per-column fold terms that k_fc2 fills while its first stages load.
-constexpr int LAYER_RES_SLICE = 64 * 68 * 4;
-constexpr int LAYER_ROWSTAT = LayerCfg::NW * LAYER_RES_SLICE;  // byte offset of the per-row statistics
-constexpr int LAYER_SMEM = LAYER_ROWSTAT + 4096;                 // 2 KB row statistics + 2 KB column terms
-static_assert(LAYER_ROWSTAT >= LayerCfg::LDS, "row statistics sit past the main-loop stages");
-static_assert(LAYER_SMEM <= 160 * 1024, "layer kernels fit the LDS");
-static_assert(LayerCfg::NW * 128 * 68 * 2 <= LAYER_ROWSTAT, "v transpose slices fit");
+// Shared memory of the layer kernels: the main-loop stages, reused by the epilogues (one WM x 68 fp32 residual slice
+// per wave, one [WN][WM + 4] bf16 transpose slice per wave, or the fc1 h tile), then the per-row statistics and
+// per-column fold terms that k_fc2 fills while its first stages load.
+template <class C>
+struct LayerMem {
+    static constexpr int PC = C::WN < 64 ? C::WN : 64;             // columns of a residual pass
+    static constexpr int LD = PC + 4;                              // floats per row of a residual slice
+    static constexpr int SLICE = C::WM * LD * 4;
+    static constexpr int TRLD = C::WM + 4;                         // halves per row of a transpose slice
+    static constexpr int TRSLICE = C::WN * TRLD * 2;
+    static constexpr int EPI = C::NW * (SLICE > TRSLICE ? SLICE : TRSLICE);
+    static constexpr int LOOP = C::LDS > C::LDS_SP ? C::LDS : C::LDS_SP;
+    static constexpr int ROWSTAT = EPI > LOOP ? EPI : LOOP;        // byte offset of the per-row statistics
+    static constexpr int SMEM = ROWSTAT + 8 * (C::BM + C::BN);     // row statistics, then column terms
+    static_assert(SMEM <= 160 * 1024, "layer kernels fit the LDS");
+};
 
 __device__ __forceinline__ uint32_t pk_bf16(float a, float b)
 {
@@ -43,7 +54,6 @@ __device__ __forceinline__ void layer_mainloop(const uint8_t *A, int lda, const 
                                                int n0, uint8_t *smem, v4f (&acc)[C::TM][C::TN], Pre pre = Pre(),
                                                int Nlive = -1)
 {
-    static_assert(!SP || C::LDS_SP <= LAYER_ROWSTAT, "sparse stages end before the row statistics");
     static_assert(!(SP && TR), "the sparse tile comes transposed from bs_mainloop_sp_t");
     if constexpr (SP) bs_mainloop_sp<C>(A, lda, sa, lds, w, wx, ws, rows, Npad, K, m0, n0, smem, acc, pre, Nlive);
     else bs_mainloop<C, Pre, true, TR>(A, lda, sa, lds, w, ws, rows, Npad, K, m0, n0, smem, acc, pre, Nlive);
@@ -58,16 +68,6 @@ __device__ __forceinline__ void layer_tile(int M, int N, int &m0, int &n0)
     n0 = tn * C::BN;
 }
 
-// Residual update x = f16(x + y) of a wave's 64 x (16 TN) tile, y in the MFMA C layout, in passes of 64 columns.
-// The wave parks 64 x 64 of y in its own LDS slice (row stride 68 floats: the 64 lanes of one store hit 64 different
-// banks), then each lane updates 8 consecutive halves with one 16-byte load and store, so one wave instruction
-// covers 8 rows of 128 bytes. Every x load of the tile is issued before the first store (one memory round trip for
-// the whole update), through a buffer descriptor that ends at row `rows`: rows past it load zero and their stores
-// are dropped, with no branch between the loads.
-struct ResIdentity {
-    __device__ __forceinline__ float operator()(int, int, int, float v) const { return v; }
-};
-
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
 // x + y for the fp16 x in the low (HI = 0) or high (HI = 1) half of a word and an fp32 y: one v_fma_mix_f32,
@@ -81,99 +81,82 @@ __device__ __forceinline__ float h_add(uint32_t xw, float y)
     return r;
 }
 
-// f(i, j, r, y) maps each accumulator to the value added (row m0 + mw + 16 i + 4 (lane >> 4) + r, column tile j).
-template <class C, class F = ResIdentity>
-__device__ __forceinline__ void residual_add(uint8_t *slices, v4f (&y)[C::TM][C::TN], uint16_t *__restrict__ x,
-                                             int mw, int nw, int rows, F f = F())
-{
-    static_assert(C::TM == 4 && C::TN % 4 == 0, "64-row wave tiles, whole 64-column passes");
-    constexpr int NP = C::TN / 4;
-    float *tr = (float *)(slices + (threadIdx.x >> 6) * LAYER_RES_SLICE);
-    const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
-    const int rs = lane >> 3, ch = lane & 7;
-    const __amdgpu_buffer_rsrc_t rx = buf_rsrc(x, (uint32_t)rows * XT_D * 2u);
-    const uint32_t off0 = (uint32_t)(((mw + rs) * XT_D + nw + 8 * ch) * 2);
-    v4u xv[NP][8];
-#pragma unroll
-    for (int pass = 0; pass < NP; pass++)
-#pragma unroll
-        for (int it = 0; it < 8; it++)
-            xv[pass][it] = __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(off0 + (uint32_t)((8 * it * XT_D + 64 * pass) * 2)), 0, 0);
-#pragma unroll
-    for (int pass = 0; pass < NP; pass++) {
-        if (pass) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the previous pass's slice reads are done
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-#pragma unroll
-                for (int r = 0; r < 4; r++)
-                    tr[(16 * i + 4 * g + r) * 68 + 16 * j + c16] = f(i, 4 * pass + j, r, y[i][4 * pass + j][r]);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slice is the wave's own: no block barrier needed
-#pragma unroll
-        for (int it = 0; it < 8; it++) {
-            const int rr = 8 * it + rs;
-            const float4 a = *(const float4 *)(tr + rr * 68 + 8 * ch), b = *(const float4 *)(tr + rr * 68 + 8 * ch + 4);
-            const v4u v = xv[pass][it];
-            v4u o;
-            o[0] = pk_f16(h_add<0>(v[0], a.x), h_add<1>(v[0], a.y));
-            o[1] = pk_f16(h_add<0>(v[1], a.z), h_add<1>(v[1], a.w));
-            o[2] = pk_f16(h_add<0>(v[2], b.x), h_add<1>(v[2], b.y));
-            o[3] = pk_f16(h_add<0>(v[3], b.z), h_add<1>(v[3], b.w));
-            __builtin_amdgcn_raw_buffer_store_b128(o, rx, (int)(off0 + (uint32_t)((8 * it * XT_D + 64 * pass) * 2)), 0, 0);
-        }
-    }
-}
-
-// residual_add for a transposed tile (the sparse main loop's, or bs_mainloop's with TR): y(jn, im) gives the four
-// values added to row mw + 16 im + (lane & 15), columns nw + 16 jn + 4 (lane >> 4) + r. The same update, with the
-// tile parked in the slice by one 16-byte store per (m tile, n tile) (row stride 68 floats: the 16 rows of one store
-// group start 4 banks apart).
+// Residual update x = f16(x + y) of a wave's WM x WN tile, transposed as bs_mainloop's TR and the sparse main loop
+// leave it: y(jn, im) gives the four values added to row mw + 16 im + (lane & 15), columns
+// nw + 16 jn + 4 (lane >> 4) + r. In passes of PC = 64 columns (32 for a 32-column tile) the wave parks its y in its
+// own LDS slice by one 16-byte store per (m tile, n tile) (rows of PC + 4 floats: the 16 rows of one store group start
+// 4 banks apart), then each lane updates 8 consecutive halves with one 16-byte load and store, so one wave
+// instruction covers whole rows of the pass. Every x load of the tile is issued before the first store (one memory
+// round trip for the whole update), through a buffer descriptor that ends at row `rows`: rows past it load zero and
+// their stores are dropped, with no branch between the loads.
 template <class C, class Y>
 __device__ __forceinline__ void residual_add_t(uint8_t *slices, Y y, uint16_t *__restrict__ x, int mw, int nw, int rows)
 {
-    static_assert(C::TM == 4 && C::TN % 4 == 0, "64-row wave tiles, whole 64-column passes");
-    constexpr int NP = C::TN / 4;
-    float *tr = (float *)(slices + (threadIdx.x >> 6) * LAYER_RES_SLICE);
+    using S = LayerMem<C>;
+    constexpr int NP = C::WN / S::PC, LPR = S::PC / 8, RPI = 64 / LPR, NI = C::WM / RPI;  // lanes a row, rows a store
+    float *tr = (float *)(slices + (threadIdx.x >> 6) * S::SLICE);
     const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
-    const int rs = lane >> 3, ch = lane & 7;
+    const int rs = lane / LPR, ch = lane % LPR;
     const __amdgpu_buffer_rsrc_t rx = buf_rsrc(x, (uint32_t)rows * XT_D * 2u);
     const uint32_t off0 = (uint32_t)(((mw + rs) * XT_D + nw + 8 * ch) * 2);
-    v4u xv[NP][8];
+    v4u xv[NP][NI];
 #pragma unroll
     for (int pass = 0; pass < NP; pass++)
 #pragma unroll
-        for (int it = 0; it < 8; it++)
-            xv[pass][it] = __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(off0 + (uint32_t)((8 * it * XT_D + 64 * pass) * 2)), 0, 0);
+        for (int it = 0; it < NI; it++)
+            xv[pass][it] = __builtin_amdgcn_raw_buffer_load_b128(rx, (int)(off0 + (uint32_t)((RPI * it * XT_D + S::PC * pass) * 2)), 0, 0);
 #pragma unroll
     for (int pass = 0; pass < NP; pass++) {
         if (pass) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the previous pass's slice reads are done
 #pragma unroll
-        for (int im = 0; im < 4; im++)
+        for (int im = 0; im < C::TM; im++)
 #pragma unroll
-            for (int jq = 0; jq < 4; jq++) {
-                const v4f v = y(4 * pass + jq, im);
-                *(float4 *)(tr + (16 * im + c16) * 68 + 16 * jq + 4 * g) = make_float4(v[0], v[1], v[2], v[3]);
+            for (int jq = 0; jq < S::PC / 16; jq++) {
+                const v4f v = y(S::PC / 16 * pass + jq, im);
+                *(float4 *)(tr + (16 * im + c16) * S::LD + 16 * jq + 4 * g) = make_float4(v[0], v[1], v[2], v[3]);
             }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slice is the wave's own: no block barrier needed
 #pragma unroll
-        for (int it = 0; it < 8; it++) {
-            const int rr = 8 * it + rs;
-            const float4 a = *(const float4 *)(tr + rr * 68 + 8 * ch), b = *(const float4 *)(tr + rr * 68 + 8 * ch + 4);
+        for (int it = 0; it < NI; it++) {
+            const int rr = RPI * it + rs;
+            const float4 a = *(const float4 *)(tr + rr * S::LD + 8 * ch), b = *(const float4 *)(tr + rr * S::LD + 8 * ch + 4);
             const v4u v = xv[pass][it];
             v4u o;
             o[0] = pk_f16(h_add<0>(v[0], a.x), h_add<1>(v[0], a.y));
             o[1] = pk_f16(h_add<0>(v[1], a.z), h_add<1>(v[1], a.w));
             o[2] = pk_f16(h_add<0>(v[2], b.x), h_add<1>(v[2], b.y));
             o[3] = pk_f16(h_add<0>(v[3], b.z), h_add<1>(v[3], b.w));
-            __builtin_amdgcn_raw_buffer_store_b128(o, rx, (int)(off0 + (uint32_t)((8 * it * XT_D + 64 * pass) * 2)), 0, 0);
+            __builtin_amdgcn_raw_buffer_store_b128(o, rx, (int)(off0 + (uint32_t)((RPI * it * XT_D + S::PC * pass) * 2)), 0, 0);
         }
     }
 }
 
-static inline unsigned layer_grid(int rows, int N, int BM, int BN)
+template <class C>
+static inline unsigned layer_grid(int rows, int N)
 {
-    return (unsigned)(((rows + BM - 1) / BM) * ((N + BN - 1) / BN));
+    return (unsigned)(((rows + C::BM - 1) / C::BM) * ((N + C::BN - 1) / C::BN));
+}
+
+// f(C{}) with the tile configuration C of a 1024-column GEMM (attention out-projection, fc2) over `rows` rows, K deep.
+// 256 x 256 tiles read each operand least and win once they fill the CUs, but give only 4 tiles per 256 rows; a K step
+// costs them about 1.35 us against 0.5-0.9 for the smaller ones, so a grid that leaves CUs idle is better cut finer.
+//  - 64 x 128 while one round of two blocks per CU holds them (rows <= 4096). us, 256 x 256 -> 64 x 128:
+//    K = 1024: 14.8 -> 5.3 at 1025 rows, 15.1 -> 6.9 at 2050; K = 2816: 32.6 -> 10.8 and 34.6 -> 15.4
+//    (128 x 128: 6.9, 7.4; 19.4, 20.5);
+//  - 128 x 128 while one round of two blocks per CU holds them (rows <= 8192): K = 2816 35.6 -> 22.5 at 4100 and
+//    36.6 -> 25.3 at 6150 (64 x 128: 26.1, 33.1); K = 1024 15.7 -> 10.0 and 17.0 -> 11.9;
+//  - above that 256 x 256 (K = 2816: 37.3 against 42.3 at 8200, 66.3 against 68.4 at 16400; K = 4736: 55.8 against
+//    67.8 at 10368), except at K <= 1024 where the whole 256 x 256 tiles leave a last round at most half full (or fill
+//    the rounds exactly and a partial row tile follows): 18.3 -> 16.9 at 8200, 31.9 -> 28.2 at 16400, 37.1 -> 34.5
+//    at 20736, 52.2 -> 46.9 at 32800 (a last round fuller than that: 18.9 against 19.3 at 10250, 44.0 against 48.9 at
+//    31104).
+template <class F>
+static inline void with_res_cfg(int rows, int K, F f)
+{
+    const int tail = rows / LayerCfg::BM * (XT_D / LayerCfg::BN) % 256;  // whole 256 x 256 tiles of the last round
+    if (rows <= 4096) f(LayerSml{});
+    else if (rows <= 8192 || (K <= XT_D && tail <= 128 && (tail || rows % LayerCfg::BM))) f(LayerMid{});
+    else f(LayerCfg{});
 }
 
 #define XT_ALIGNED(p) ((((uintptr_t)(p)) & 15) == 0)

@@ -52,7 +52,7 @@ __global__ void __launch_bounds__(LayerCfg::NT) k_px_qkv(const uint8_t *__restri
                                                         uint16_t *__restrict__ vt, int rows)
 {
     using C = LayerCfg;
-    __shared__ __attribute__((aligned(16))) uint8_t smem[LAYER_SMEM];
+    __shared__ __attribute__((aligned(16))) uint8_t smem[LayerMem<C>::SMEM];
     v4f acc[C::TM][C::TN];
     int m0, n0, wm0, wn0;
     layer_tile<C>(rows, 3 * XT_D, m0, n0);
@@ -132,21 +132,19 @@ __global__ void __launch_bounds__(LayerCfg::NT) k_px_qkv(const uint8_t *__restri
 // k_pfc2). The reference rounds (x + alpha acc) + b in fp32 (px_kernels.cu:178); here acc + b is formed first: the
 // two orders differ by at most one fp32 rounding before the fp16 store.
 // ---------------------------------------------------------------------------------------------------------------
-template <bool SP, int K>
-__global__ void __launch_bounds__(LayerCfg::NT) k_px_res(const uint8_t *__restrict__ a8, const float *__restrict__ as,
-                                                        int lds, const uint8_t *__restrict__ w,
-                                                        const uint32_t *__restrict__ wx, const float *__restrict__ ws,
+template <class C, int K>
+__global__ void __launch_bounds__(C::NT) k_px_res(const uint8_t *__restrict__ a8, const float *__restrict__ as,
+                                                        int lds, const uint8_t *__restrict__ w, const float *__restrict__ ws,
                                                         const float *__restrict__ bias, uint16_t *__restrict__ x,
                                                         int rows)
 {
-    using C = LayerCfg;
-    __shared__ __attribute__((aligned(16))) uint8_t smem[LAYER_SMEM];
+    __shared__ __attribute__((aligned(16))) uint8_t smem[LayerMem<C>::SMEM];
     v4f acc[C::TM][C::TN];
     int m0, n0, wm0, wn0;
     layer_tile<C>(rows, XT_D, m0, n0);
     args_resident(bias, x, lds, rows);
     // the tile transposed (TR): lane (g, c16) holds columns n0 + wn0 + 16 j + 4 g + r, one 16-byte bias load per j
-    layer_mainloop<C, SP, BsNoPre, true>(a8, K, as, lds, w, wx, ws, rows, XT_D, K, m0, n0, smem, acc);
+    layer_mainloop<C, false, BsNoPre, true>(a8, K, as, lds, w, nullptr, ws, rows, XT_D, K, m0, n0, smem, acc);
     bs_wave_origin<C>(wm0, wn0);
     const int g = (threadIdx.x & 63) >> 4;
     float4 b4[C::TN];
@@ -175,7 +173,7 @@ __global__ void __launch_bounds__(LayerCfg::NT) k_px_fc1(const uint8_t *__restri
 {
     using C = LayerCfg;
     static_assert(C::TM == 4 && C::TN == 8 && C::WN == 128, "a wave tile is 64 rows x one 128-unit scale block");
-    __shared__ __attribute__((aligned(16))) uint8_t smem[LAYER_SMEM];
+    __shared__ __attribute__((aligned(16))) uint8_t smem[LayerMem<C>::SMEM];
     v4f acc[C::TM][C::TN];
     int m0, n0, wm0, wn0;
     layer_tile<C>(rows, PX_HID, m0, n0);
@@ -215,7 +213,7 @@ __global__ void __launch_bounds__(LayerCfg::NT) k_px_fc1(const uint8_t *__restri
         const int m = m0 + wm0 + 16 * i + c16;
         if (g == 0 && m < rows) ms[(size_t)blk * lds + m] = sc;
     }
-    float *tr = (float *)(smem + (threadIdx.x >> 6) * LAYER_RES_SLICE);
+    float *tr = (float *)(smem + (threadIdx.x >> 6) * LayerMem<C>::SLICE);
     const __amdgpu_buffer_rsrc_t rm = buf_rsrc(m8, (uint32_t)rows * PX_HID);
     const int rsub = lane >> 3, ch = lane & 7;
 #pragma unroll
@@ -253,7 +251,7 @@ extern "C" int px_k_qkv(const void *h8, const float *hs, int lds, const void *w,
     if (L <= 0 || L % 64 || rows % L) return xt_fail("px_k_qkv", "L must be a positive multiple of 64 dividing rows");
     if (!XT_ALIGNED(h8) || !XT_ALIGNED(w) || ((uintptr_t)bias & 7) || ((uintptr_t)cs & 7))
         return xt_fail("px_k_qkv", "h8 and w must be 16-byte aligned, bias and cs 8-byte aligned");
-    hipLaunchKernelGGL(k_px_qkv<false>, dim3(layer_grid(rows, 3 * XT_D, LayerCfg::BM, LayerCfg::BN)),
+    hipLaunchKernelGGL(k_px_qkv<false>, dim3(layer_grid<LayerCfg>(rows, 3 * XT_D)),
                        dim3(LayerCfg::NT), 0, (hipStream_t)stream, (const uint8_t *)h8, hs, lds, (const uint8_t *)w,
                        (const uint32_t *)nullptr, ws, bias, cs, L, (uint16_t *)q, (uint16_t *)k, (uint16_t *)vt, rows);
     return xt_check("px_k_qkv");
@@ -265,9 +263,11 @@ static int px_res_launch(const char *what, const void *a8, const float *as, int 
 {
     if (layer_rows_ok(what, rows, lds)) return -1;
     if (!XT_ALIGNED(a8) || !XT_ALIGNED(w)) return xt_fail(what, "a8 and w must be 16-byte aligned");
-    hipLaunchKernelGGL((k_px_res<false, K>), dim3(layer_grid(rows, XT_D, LayerCfg::BM, LayerCfg::BN)), dim3(LayerCfg::NT),
-                       0, (hipStream_t)stream, (const uint8_t *)a8, as, lds, (const uint8_t *)w,
-                       (const uint32_t *)nullptr, ws, bias, (uint16_t *)x, rows);
+    with_res_cfg(rows, K, [&](auto c) {
+        using C = decltype(c);
+        hipLaunchKernelGGL((k_px_res<C, K>), dim3(layer_grid<C>(rows, XT_D)), dim3(C::NT), 0, (hipStream_t)stream,
+                           (const uint8_t *)a8, as, lds, (const uint8_t *)w, ws, bias, (uint16_t *)x, rows);
+    });
     return xt_check(what);
 }
 
@@ -290,7 +290,7 @@ extern "C" int px_k_fc1(const void *h8, const float *hs, int lds, const void *w,
     if (!XT_ALIGNED(h8) || !XT_ALIGNED(w) || ((uintptr_t)m8 & 7))
         return xt_fail("px_k_fc1", "h8 and w must be 16-byte aligned, m8 8-byte aligned");
     auto kern = rs ? k_px_fc1<false, true> : k_px_fc1<false, false>;  // the multiply only where rs is given
-    hipLaunchKernelGGL(kern, dim3(layer_grid(rows, PX_HID, LayerCfg::BM, LayerCfg::BN)), dim3(LayerCfg::NT), 0,
+    hipLaunchKernelGGL(kern, dim3(layer_grid<LayerCfg>(rows, PX_HID)), dim3(LayerCfg::NT), 0,
                        (hipStream_t)stream, (const uint8_t *)h8, hs, lds, (const uint8_t *)w, (const uint32_t *)nullptr,
                        ws, bias, rs, (uint8_t *)m8, ms, rows);
     return xt_check("px_k_fc1");
