@@ -2,7 +2,8 @@
 // (src/engine/kern_common.cuh:403-543) on CDNA4 bf16 matrix cores, with the output packed to E4M3 1x128 blocks
 // for the out-projection.
 //
-// Per (image, head pair, 128-query block): 8 waves, waves 0-3 on head 2p and 4-7 on head 2p+1, 32 queries each.
+// Per (image, head pair, block of 128 or 64 queries): 8 or 4 waves, the first half on head 2p, the others on head
+// 2p+1, 32 queries each.
 // Scores are computed transposed, S^T = K Q^T (v_mfma_f32_32x32x16_bf16: A = 32 keys, B = 32 queries), so every lane
 // owns one query and 16 keys of a 32-key tile. Lane group g = lane >> 5 holds accumulator rows 8j + 4g + i; the K
 // fragment of lane l is read from key row pi(l & 31) with pi(8j + 4g + i) = 16(j >> 1) + 8g + 4(j & 1) + i, which
@@ -20,7 +21,6 @@
 #include "gemm_core.h"
 #include "xt_abi.h"
 
-#define FA_QB 128                    // queries per block
 #define FA_KT 64                     // keys per LDS tile
 #define FA_TILE (FA_KT * 128)        // bytes of one K or V^T tile of one head
 #define FA_STAGE (4 * FA_TILE)       // K head 0 | K head 1 | V^T head 0 | V^T head 1
@@ -37,6 +37,12 @@ __device__ __forceinline__ v8bf frag_bf(const uint8_t *tile, int row, int chunk)
     return __builtin_bit_cast(v8bf, *(const uint4 *)(tile + swz_kv(row, chunk)));
 }
 
+// 1 KB to LDS: lane l's 16 bytes at voff + soff land at dst + 16 l
+__device__ __forceinline__ void kv_dma(__amdgpu_buffer_rsrc_t r, uint8_t *dst, uint32_t voff, uint32_t soff)
+{
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void *)dst, 16, voff, soff, 0, 0);
+}
+
 typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
 #define kOnes2 (v2bf{(__bf16)1.0f, (__bf16)1.0f})
 
@@ -47,51 +53,51 @@ __device__ __forceinline__ v8bf pack_p(const v16f &s, int base)
     return __builtin_convertvector(f, v8bf);
 }
 
-// One block per (query block of 128, head pair, sequence): sequences of T tokens, q / k rows and v^T columns padded to
+// One block per (query block of 32 QT, head pair, sequence): sequences of T tokens, q / k rows and v^T columns padded to
 // TP >= T rounded up to 64 (rows past T read as data must be finite; keys past T are masked). When T = 64 n + 1
 // (n > 0: the wd model's 1025 tokens) the last key is not streamed as a 17th tile of one key: each lane adds it after
 // the n tiles from global memory (one score, one weight, 32 products).
-template <int DBG>
-__global__ void __launch_bounds__(512) k_flash(const uint16_t *__restrict__ q, const uint16_t *__restrict__ k,
+template <int QT, int DBG>
+__global__ void __launch_bounds__(128 * QT) k_flash(const uint16_t *__restrict__ q, const uint16_t *__restrict__ k,
                                                const uint16_t *__restrict__ vt, uint8_t *__restrict__ o8,
                                                float *__restrict__ os, int lds, float *__restrict__ o32, int T, int TP)
 {
-    __shared__ __attribute__((aligned(16))) uint8_t smem[2 * FA_STAGE + 8 * 32 * 4];
+    constexpr int QB = 32 * QT, LPW = 16 / QT;  // queries per block, 1 KB loads per wave and stage
+    __shared__ __attribute__((aligned(16))) uint8_t smem[2 * FA_STAGE + 2 * QT * 32 * 4];
     float *xamax = (float *)(smem + 2 * FA_STAGE);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 5, l32 = lane & 31;
     // 1-D grid, XCD-aware: block i runs on XCD i % 8, and the query blocks of one (sequence, head pair) share its K
     // and V^T, so they all take the same i % 8 (consecutive i / 8): their K / V^T tiles are fetched into one XCD's L2
     // once instead of into every XCD's
-    const int nqb = (T + FA_QB - 1) / FA_QB, bi = blockIdx.x >> 3, grp = 8 * (bi / nqb) + (blockIdx.x & 7);
+    const int nqb = (T + QB - 1) / QB, bi = blockIdx.x >> 3, grp = 8 * (bi / nqb) + (blockIdx.x & 7);
     const int qb = bi - (bi / nqb) * nqb, hp = grp & (XT_NH / 2 - 1), b = grp / (XT_NH / 2);
-    const int hsel = w >> 2, qt = w & 3;
+    const int hsel = w / QT, qt = w % QT;
     const int head = 2 * hp + hsel;
-    const int q0 = qb * FA_QB + 32 * qt;
+    const int q0 = qb * QB + 32 * qt;
     const bool active = q0 < T;
     const bool xkey = (T & (FA_KT - 1)) == 1 && T > FA_KT;   // the last key alone, after the tiles
     const int nkt = xkey ? T / FA_KT : (T + FA_KT - 1) / FA_KT;
 
-    // operand loads: per stage 32 x 1 KB, 4 per wave: waves 0-1 K head 2p, 2-3 K head 2p+1, 4-5 V^T head 2p, 6-7 V^T
-    // head 2p+1 (K: 8 contiguous KB per head; V^T: 64 rows of 128 B, stride TP). The per-lane offsets are fixed; the
+    // operand loads: per stage 32 x 1 KB, LPW per wave in this order: K head 2p, K head 2p+1, V^T head 2p, V^T head
+    // 2p+1, 8 each (K: 8 contiguous KB per head; V^T: 64 rows of 128 B, stride TP). The per-lane offsets are fixed; the
     // key tile moves only the scalar offset (8 KB of K or 128 B of V^T per tile).
     const size_t hbase0 = ((size_t)b * XT_NH + 2 * hp) * TP * XT_HD;  // elements, head 2p
     const __amdgpu_buffer_rsrc_t rk = buf_rsrc(k + hbase0, 2u * (uint32_t)TP * XT_HD * 2u);
     const __amdgpu_buffer_rsrc_t rv = buf_rsrc(vt + hbase0, 2u * (uint32_t)TP * XT_HD * 2u);
     const int wu = __builtin_amdgcn_readfirstlane(w);
-    const bool dk = wu < 4;
-    const int hh = (wu >> 1) & 1, r8 = lane >> 3;
+    const bool dk = wu < QT;
+    const int hh = (wu * LPW >> 3) & 1, r8 = lane >> 3;
     const uint32_t kstep = dk ? FA_KT * 128u : FA_KT * 2u;
-    uint32_t voff[4];
+    uint32_t voff[LPW];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {  // lane: LDS row rowb, slot lane & 7, which holds chunk (lane & 7) ^ ((rowb >> 1) & 7)
-        const int rowb = 8 * ((wu * 4 + i) & 7) + r8, ch = (lane & 7) ^ ((rowb >> 1) & 7);
+    for (int i = 0; i < LPW; i++) {  // lane: LDS row rowb, slot lane & 7, which holds chunk (lane & 7) ^ ((rowb >> 1) & 7)
+        const int rowb = 8 * ((wu * LPW + i) & 7) + r8, ch = (lane & 7) ^ ((rowb >> 1) & 7);
         voff[i] = dk ? (uint32_t)((hh * TP + rowb) * 128 + ch * 16) : (uint32_t)((hh * XT_HD + rowb) * TP * 2 + ch * 16);
     }
     auto issue = [&](uint8_t *st, int kt) {
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(dk ? rk : rv, (lds_void *)(st + 1024 * (wu * 4 + i)), 16, voff[i],
-                                                     (uint32_t)kt * kstep, 0, 0);
+        for (int i = 0; i < LPW; i++)
+            kv_dma(dk ? rk : rv, st + 1024 * (wu * LPW + i), voff[i], (uint32_t)kt * kstep);
     };
 
     // Q fragments (B operand of S^T): query q0 + l32, dims 16 step + 8 g .. + 8
@@ -304,7 +310,7 @@ __global__ void __launch_bounds__(512) k_flash(const uint16_t *__restrict__ q, c
     if (lane < 32) xamax[w * 32 + lane] = amax;
     __syncthreads();
     if (!active) return;
-    amax = __builtin_fmaxf(amax, xamax[(w ^ 4) * 32 + l32]);
+    amax = __builtin_fmaxf(amax, xamax[(w ^ QT) * 32 + l32]);
     const float sc = block_scale(amax), inv = block_scale_inv(sc);
     const int query = q0 + l32;
     if (query >= T) return;
@@ -325,6 +331,21 @@ __global__ void __launch_bounds__(512) k_flash(const uint16_t *__restrict__ q, c
     if (hsel == 0 && g == 0) os[(size_t)hp * lds + m] = sc;
 }
 
+// Queries per block: 128 (QT = 4 query tiles of 32 per head, two waves per SIMD), or 64 while those blocks get a CU
+// each: a wave alone on its SIMD runs a key tile in 1.2 us, one of two in 1.4. us, 128 -> 64 queries: 23.8 -> 20.4 for
+// one sequence of 1025 (72 -> 136 blocks), 9.9 -> 8.3 for one of 200; with more blocks than CUs the halved reuse of
+// the K and V^T stages loses (two sequences of 1025: 24.8 -> 28.1; 18 of 576: 38.3 -> 48.0).
+template <int N>
+struct FaQt {
+    static constexpr int value = N;
+};
+template <class F>
+static void with_flash_qt(int nseq, int T, F f)
+{
+    if ((size_t)((T + 63) / 64) * (XT_NH / 2) * nseq <= 256) f(FaQt<2>{});
+    else f(FaQt<4>{});
+}
+
 static int flash_launch(const char *what, const void *q, const void *k, const void *vt, void *o8, float *os, int lds,
                         int nseq, int T, int TP, float *o32, void *stream)
 {
@@ -333,14 +354,17 @@ static int flash_launch(const char *what, const void *q, const void *k, const vo
     if ((((uintptr_t)q) | ((uintptr_t)k) | ((uintptr_t)vt) | ((uintptr_t)o8)) & 15)
         return xt_fail(what, "q, k, vt, o8 must be 16-byte aligned");
     static_assert(XT_NH / 2 == 8, "the XCD-aware block order groups 8 head pairs per sequence");
-    if ((size_t)(T + FA_QB - 1) / FA_QB * (XT_NH / 2) * nseq > 0x7fffffffu) return xt_fail(what, "grid too large");
-    const dim3 grid((T + FA_QB - 1) / FA_QB * (XT_NH / 2) * nseq);
-    if (o32)
-        hipLaunchKernelGGL(k_flash<1>, grid, dim3(512), 0, (hipStream_t)stream, (const uint16_t *)q, (const uint16_t *)k,
-                           (const uint16_t *)vt, (uint8_t *)o8, os, lds, o32, T, TP);
-    else
-        hipLaunchKernelGGL(k_flash<0>, grid, dim3(512), 0, (hipStream_t)stream, (const uint16_t *)q, (const uint16_t *)k,
-                           (const uint16_t *)vt, (uint8_t *)o8, os, lds, o32, T, TP);
+    if ((size_t)((T + 31) / 32) * (XT_NH / 2) * nseq > 0x7fffffffu) return xt_fail(what, "grid too large");
+    with_flash_qt(nseq, T, [&](auto c) {
+        constexpr int QT = decltype(c)::value;
+        const dim3 grid((T + 32 * QT - 1) / (32 * QT) * (XT_NH / 2) * nseq);
+        if (o32)
+            hipLaunchKernelGGL((k_flash<QT, 1>), grid, dim3(128 * QT), 0, (hipStream_t)stream, (const uint16_t *)q,
+                               (const uint16_t *)k, (const uint16_t *)vt, (uint8_t *)o8, os, lds, o32, T, TP);
+        else
+            hipLaunchKernelGGL((k_flash<QT, 0>), grid, dim3(128 * QT), 0, (hipStream_t)stream, (const uint16_t *)q,
+                               (const uint16_t *)k, (const uint16_t *)vt, (uint8_t *)o8, os, lds, o32, T, TP);
+    });
     return xt_check(what);
 }
 
