@@ -420,92 +420,124 @@ __global__ void __launch_bounds__(256) k_head(const uint8_t *__restrict__ pq, co
 // ---------------------------------------------------------------------------------------------------------------
 // k_pe: patch embedding in fp16 with fp32 accumulation (v_mfma_f32_16x16x32_f16) and the position add fused
 // (k_pe + k_embed, eva_kernels.cu:21-33, 126-130): x[1025 b + 1 + p] = f16(in[1024 b + p] . pe^T + pos[1 + p]),
-// x[1025 b] = f16(pos[0]) (pos carries cls and the conv bias, export_eva.py:76-80). Block 128 patches x 128
-// columns, 4 waves of 64 x 64, K = 592 in steps of 64 halves (the last step holds 16; the rest is zeroed).
-// ---------------------------------------------------------------------------------------------------------------
+// x[1025 b] = f16(pos[0]) (pos carries cls and the conv bias, export_eva.py:76-80). K = 592 in steps of 64 halves:
+// rows of 128 bytes, as the E4M3 operands of the layer GEMMs, brought into LDS the same way (16-byte chunk c of row r
+// at (c + r) & 7, C::NS stages, counted waits); the last step holds 16 halves, and the lanes whose chunk lies past
+// them load an out-of-range offset (zero). The tile is transposed (weights as the MFMA's A operand), parked in the
+// wave's slice of shared memory and leaves as whole 128-byte rows. Tile sizes: with_pe_cfg.
 // PX: the PixAI patch GEMM (px_kernels.cu:133-138 k_ppe) instead: x[m] = f16(in[m] . pe^T) for window-major token rows
 // m (no cls, no position: k_px_pembed adds it before its LayerNorm), rows a multiple of 128.
-template <bool PX>
-__global__ void __launch_bounds__(256) k_pe(const uint16_t *__restrict__ in, const uint16_t *__restrict__ pe,
-                                            const float *__restrict__ pos, uint16_t *__restrict__ x, int nb)
+// ---------------------------------------------------------------------------------------------------------------
+typedef float v4f_e __attribute__((ext_vector_type(4), aligned(4)));     // 16 bytes of a buffer aligned to its
+typedef unsigned v4u_e __attribute__((ext_vector_type(4), aligned(2)));  // elements only (pos fp32, x fp16)
+template <class C, bool PX>
+__global__ void __launch_bounds__(C::NT) k_pe(const uint16_t *__restrict__ in, const uint16_t *__restrict__ pe,
+                                              const float *__restrict__ pos, uint16_t *__restrict__ x, int rows)
 {
-    __shared__ __attribute__((aligned(16))) uint8_t smem[2 * 128 * 128];  // A | B tile of one K step
-    const int m0 = blockIdx.y * 128, n0 = blockIdx.x * 128, t = threadIdx.x;
-    const int lane = t & 63, w = t >> 6, g = lane >> 4, r16 = lane & 15;
-    const int wm0 = (w >> 1) * 64, wn0 = (w & 1) * 64;
-    v4f acc[4][4];
+    using S = LayerMem<C>;
+    constexpr int STAGE = C::A_BYTES + C::B_BYTES, KB = (XT_K0P + 63) / 64, LPS = C::LA + C::LB;
+    constexpr int LAST = XT_K0P % 64 / 8;  // 16-byte chunks of the last K step
+    constexpr uint32_t LDB = XT_K0P * 2;
+    constexpr int SLICES = C::NW * S::SLICE;
+    static_assert(LAST > 0 && C::BM <= 128, "a partial last step; row tiles divide the 128-row granule of every caller");
+    __shared__ __attribute__((aligned(16))) uint8_t smem[SLICES > C::NS * STAGE ? SLICES : C::NS * STAGE];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int m0, n0, wm0, wn0;
+    layer_tile<C>(rows, XT_D, m0, n0);  // XCD-aware: an XCD's blocks share their rows of `in` in its L2
+    bs_wave_origin<C>(wm0, wn0);
+    args_resident(pos, x);
+    const v4i ra = buf_desc(in + (size_t)m0 * XT_K0P, C::BM * LDB), rb = buf_desc(pe + (size_t)n0 * XT_K0P, C::BN * LDB);
+    const uint32_t base = lds_addr(smem);
+    uint32_t off[LPS];
+    bool tail[LPS];  // this lane's chunk lies past the last step's
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < LPS; i++) {
+        const int rl = 8 * (i < C::LA ? w * C::LA + i : w * C::LB + i - C::LA) + (lane >> 3), ch = ((lane & 7) - rl) & 7;
+        off[i] = (uint32_t)rl * LDB + 16u * ch;
+        tail[i] = ch >= LAST;
+    }
+    auto issue = [&](int stage, int kb) {
+        const uint32_t st = base + (uint32_t)stage * STAGE;
 #pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-    // stage: 128 rows x 8 chunks of 8 halves for A and B; chunks past column 592 are zero. The next K step's chunks
-    // are loaded into registers while the current step's MFMAs run.
-    uint4 va[4], vb[4];
-    auto fetch = [&](int k0) {
-#pragma unroll
-        for (int it = 0; it < 4; it++) {
-            const int idx = t + 256 * it, row = idx >> 3, ch = idx & 7, col = k0 + 8 * ch;
-            va[it] = vb[it] = make_uint4(0, 0, 0, 0);
-            if (col < XT_K0P) {
-                va[it] = *(const uint4 *)(in + (size_t)(m0 + row) * XT_K0P + col);
-                vb[it] = *(const uint4 *)(pe + (size_t)(n0 + row) * XT_K0P + col);
-            }
+        for (int i = 0; i < LPS; i++) {
+            const uint32_t o = kb == KB - 1 && tail[i] ? XT_OOR : off[i];
+            if (i < C::LA) dma16(ra, st + 1024u * (w * C::LA + i), o, (uint32_t)kb * 128u);
+            else dma16(rb, st + C::A_BYTES + 1024u * (w * C::LB + i - C::LA), o, (uint32_t)kb * 128u);
         }
     };
-    fetch(0);
-    for (int k0 = 0; k0 < XT_K0P; k0 += 64) {
+    v4f acc[C::TM][C::TN];
 #pragma unroll
-        for (int it = 0; it < 4; it++) {
-            const int idx = t + 256 * it, row = idx >> 3, ch = idx & 7;
-            *(uint4 *)(smem + swz(row, ch)) = va[it];
-            *(uint4 *)(smem + 128 * 128 + swz(row, ch)) = vb[it];
+    for (int i = 0; i < C::TM; i++)
+#pragma unroll
+        for (int j = 0; j < C::TN; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    static_assert(C::NS - 1 <= KB, "the prologue issues whole steps");
+#pragma unroll
+    for (int k = 0; k < C::NS - 1; k++) issue(k, k);
+    int cs = 0, is = C::NS - 1;
+    for (int kb = 0; kb < KB; kb++) {
+        wait_stages<C::NS - 2, LPS>(KB - 1 - kb);
+        lds_barrier();
+        if (kb + C::NS - 1 < KB) issue(is, kb + C::NS - 1);
+        const uint8_t *ta = smem + cs * STAGE, *tb = ta + C::A_BYTES;
+        typedef int v4w __attribute__((ext_vector_type(4)));
+        v8i a[C::TM];
+#pragma unroll
+        for (int i = 0; i < C::TM; i++) a[i] = ld_frag(ta, wm0 + 16 * i);
+#pragma unroll
+        for (int j = 0; j < C::TN; j++) {
+            const v8i b = ld_frag(tb, wn0 + 16 * j);
+            const v8h blo = __builtin_bit_cast(v8h, v4w{b[0], b[1], b[2], b[3]});
+            const v8h bhi = __builtin_bit_cast(v8h, v4w{b[4], b[5], b[6], b[7]});
+#pragma unroll
+            for (int i = 0; i < C::TM; i++)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                    blo, __builtin_bit_cast(v8h, v4w{a[i][0], a[i][1], a[i][2], a[i][3]}), acc[i][j], 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < C::TM; i++)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                    bhi, __builtin_bit_cast(v8h, v4w{a[i][4], a[i][5], a[i][6], a[i][7]}), acc[i][j], 0, 0, 0);
         }
-        __syncthreads();
-        if (k0 + 64 < XT_K0P) fetch(k0 + 64);
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-            v8h a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) a[i] = __builtin_bit_cast(v8h, *(const uint4 *)(smem + swz(wm0 + 16 * i + r16, 4 * s + g)));
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                b[j] = __builtin_bit_cast(v8h, *(const uint4 *)(smem + 128 * 128 + swz(wn0 + 16 * j + r16, 4 * s + g)));
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
-        __syncthreads();
+        cs = cs == C::NS - 1 ? 0 : cs + 1;
+        is = is == C::NS - 1 ? 0 : is + 1;
     }
-    const int c16 = lane & 15;
-    if constexpr (PX) {
+    lds_barrier();
+    // acc[i][j][r]: row wm0 + 16 i + (lane & 15), column wn0 + 16 j + 4 (lane >> 4) + r
+    constexpr int NP = C::WN / S::PC, LPR = S::PC / 8, RPI = 64 / LPR, NI = C::WM / RPI;  // lanes a row, rows a store
+    float *tr = (float *)(smem + w * S::SLICE);
+    const int g = lane >> 4, c16 = lane & 15, rs = lane / LPR, ch = lane % LPR;
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+    for (int pass = 0; pass < NP; pass++) {
+        const int n = n0 + wn0 + S::PC * pass + 8 * ch;
+        if (pass) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the previous pass's slice reads are done
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                uint16_t *xr = x + (size_t)(m0 + wm0 + 16 * i + 4 * g + r) * XT_D;
+        for (int i = 0; i < C::TM; i++)
 #pragma unroll
-                for (int j = 0; j < 4; j++) xr[n0 + wn0 + 16 * j + c16] = f2h(acc[i][j][r]);
+            for (int jq = 0; jq < S::PC / 16; jq++) {
+                const v4f v = acc[i][S::PC / 16 * pass + jq];
+                *(float4 *)(tr + (16 * i + c16) * S::LD + 16 * jq + 4 * g) = make_float4(v[0], v[1], v[2], v[3]);
             }
-        return;
-    }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slice is the wave's own: no block barrier needed
 #pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const int m = m0 + wm0 + 16 * i + 4 * g + r, b = m >> 10, p = m & 1023;
-            uint16_t *xr = x + ((size_t)b * XT_T + 1 + p) * XT_D;
-            const float *pr = pos + (size_t)(1 + p) * XT_D;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int n = n0 + wn0 + 16 * j + c16;
-                xr[n] = f2h(acc[i][j][r] + pr[n]);
+        for (int it = 0; it < NI; it++) {
+            const int rr = RPI * it + rs, m = m0 + wm0 + rr;
+            float4 a = *(const float4 *)(tr + rr * S::LD + 8 * ch), b = *(const float4 *)(tr + rr * S::LD + 8 * ch + 4);
+            size_t row = m;
+            if constexpr (!PX) {
+                const int img = m >> 10, p = m & 1023;
+                row = (size_t)img * XT_T + 1 + p;
+                const float *pr = pos + (size_t)(1 + p) * XT_D + n;
+                const v4f_e pa = *(const v4f_e *)pr, pb = *(const v4f_e *)(pr + 4);
+                a = make_float4(a.x + pa[0], a.y + pa[1], a.z + pa[2], a.w + pa[3]);
+                b = make_float4(b.x + pb[0], b.y + pb[1], b.z + pb[2], b.w + pb[3]);
             }
+            *(v4u_e *)(x + row * XT_D + n) = v4u_e{pk_f16(a.x, a.y), pk_f16(a.z, a.w), pk_f16(b.x, b.y), pk_f16(b.z, b.w)};
         }
-    if ((m0 & 1023) == 0 && t < 128) {  // the first patch tile of an image also writes its cls row
-        const int b = m0 >> 10, n = n0 + t;
-        x[(size_t)b * XT_T * XT_D + n] = f2h(pos[n]);
     }
+    if constexpr (!PX)
+        if ((m0 & 1023) == 0 && threadIdx.x < C::BN) {  // the first patch tile of an image also writes its cls row
+            const int n = n0 + threadIdx.x;
+            x[(size_t)(m0 >> 10) * XT_T * XT_D + n] = f2h(pos[n]);
+        }
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -675,12 +707,29 @@ extern "C" int eva_k_head(const void *pq, const float *ps, int lds, const void *
     return xt_check("eva_k_head");
 }
 
+// k_pe's tiles: 64 x 64 for up to 2048 patches (256 blocks for one image: 15.7 -> 5.0 us against the register-staged
+// 128 x 128 tiles of the version before, whose ten K steps each waited out a load; 128 x 128 tiles here 7.6), 128 x 128
+// in 8 waves beyond (us, before -> now: 22.4 -> 12.0 at 4 images, 52 -> 36 at 16, 102 -> 68 at 32; 10368 PixAI patches
+// 27.1 -> 22.2, 41472: 94 -> 74; 64 x 64: 13.6, 47.5, 89, 28.3, 101). Bound there by LDS reads (one 1 KB fragment per
+// two matrix instructions) and the 2 B store and 4 B position read per output.
+typedef BsCfg<64, 64, 2, 2, 3> PeSml;
+template <class F>
+static void with_pe_cfg(int rows, F f)
+{
+    if (rows <= 2048) f(PeSml{});
+    else f(LayerMid{});
+}
+
 extern "C" int eva_k_pe(const void *in, const void *pe, const float *pos, void *x, int nb, void *stream)
 {
     if (nb <= 0) return xt_fail("eva_k_pe", "nb must be positive");
     if (!XT_ALIGNED(in) || !XT_ALIGNED(pe)) return xt_fail("eva_k_pe", "in and pe must be 16-byte aligned");
-    hipLaunchKernelGGL(k_pe<false>, dim3(XT_D / 128, nb * XT_NP / 128), dim3(256), 0, (hipStream_t)stream,
-                       (const uint16_t *)in, (const uint16_t *)pe, pos, (uint16_t *)x, nb);
+    if (nb > (1 << 19)) return xt_fail("eva_k_pe", "at most 2^19 images");
+    with_pe_cfg(nb * XT_NP, [&](auto c) {
+        using C = decltype(c);
+        hipLaunchKernelGGL((k_pe<C, false>), dim3(layer_grid<C>(nb * XT_NP, XT_D)), dim3(C::NT), 0, (hipStream_t)stream,
+                           (const uint16_t *)in, (const uint16_t *)pe, pos, (uint16_t *)x, nb * XT_NP);
+    });
     return xt_check("eva_k_pe");
 }
 
@@ -688,7 +737,10 @@ extern "C" int px_k_pe(const void *in, const void *pe, void *x, int rows, void *
 {
     if (rows <= 0 || rows % 128) return xt_fail("px_k_pe", "rows must be a positive multiple of 128 (an even batch)");
     if (!XT_ALIGNED(in) || !XT_ALIGNED(pe)) return xt_fail("px_k_pe", "in and pe must be 16-byte aligned");
-    hipLaunchKernelGGL(k_pe<true>, dim3(XT_D / 128, rows / 128), dim3(256), 0, (hipStream_t)stream,
-                       (const uint16_t *)in, (const uint16_t *)pe, (const float *)nullptr, (uint16_t *)x, 0);
+    with_pe_cfg(rows, [&](auto c) {
+        using C = decltype(c);
+        hipLaunchKernelGGL((k_pe<C, true>), dim3(layer_grid<C>(rows, XT_D)), dim3(C::NT), 0, (hipStream_t)stream,
+                           (const uint16_t *)in, (const uint16_t *)pe, (const float *)nullptr, (uint16_t *)x, rows);
+    });
     return xt_check("px_k_pe");
 }
