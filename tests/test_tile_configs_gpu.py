@@ -91,3 +91,75 @@ def test_qkv_rows_do_not_depend_on_the_tile(dev, xt, nb, sparse):
 
     for got, ref in zip(run(nb), run(1)):
         assert torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("nb", [2, 3])
+def test_patch_embedding_does_not_depend_on_the_tile(dev, xt, nb):
+    """wd: nb images at once (64 x 64 tiles up to two, 128 x 128 from three) against each alone; PixAI: 128 nb 9 rows
+    against pieces of 128."""
+    print(f"patch embedding: {nb} images", flush=True)
+    L, P, st = xt.lib, xt.ptr, torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=dev)
+    g.manual_seed(nb)
+    x_in = torch.randn(nb * 1152, 592, generator=g, device=dev).half()
+    pe, pos = (torch.randn(D, 592, generator=g, device=dev) * 0.05).half(), torch.randn(T, D, generator=g, device=dev)
+    a, b = (torch.zeros(nb * T, D, dtype=torch.float16, device=dev) for _ in range(2))
+    assert L.eva_k_pe(P(x_in), P(pe), P(pos), P(a), nb, st) == 0
+    for i in range(nb):
+        assert L.eva_k_pe(P(x_in[1024 * i:]), P(pe), P(pos), P(b[T * i:]), 1, st) == 0
+    assert torch.equal(a, b) and a.abs().sum() > 0
+    ref = (x_in[:1024].cpu().double() @ pe.cpu().double().T + pos[1:].cpu().double()).numpy()
+    assert abs(a[1:T].cpu().double().numpy() - ref).max() <= 2.0 ** -11 * abs(ref).max() + 1e-4   # fp16 + fp32 sums
+    rows = nb * 1152
+    a, b = (torch.zeros(rows, D, dtype=torch.float16, device=dev) for _ in range(2))
+    assert L.px_k_pe(P(x_in), P(pe), P(a), rows, st) == 0
+    for r in range(0, rows, 128):
+        assert L.px_k_pe(P(x_in[r:]), P(pe), P(b[r:]), 128, st) == 0
+    assert torch.equal(a, b) and a.abs().sum() > 0
+
+
+@pytest.mark.parametrize("nseq,T_,TP", [(3, 1025, 1088), (9, 576, 576), (40, 65, 128)])
+def test_attention_does_not_depend_on_the_block(dev, xt, nseq, T_, TP):
+    """sequences at once (128 queries a block) against each alone (64 queries a block)"""
+    print(f"attention: {nseq} sequences of {T_}", flush=True)
+    L, P, st = xt.lib, xt.ptr, torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=dev)
+    g.manual_seed(T_)
+    q, k = (torch.randn(nseq, 16, TP, 64, generator=g, device=dev).bfloat16() for _ in range(2))
+    v = torch.randn(nseq, 16, 64, TP, generator=g, device=dev).bfloat16()
+    rows = nseq * T_
+
+    def run(step):
+        o8, s = torch.zeros(rows, D, dtype=U8, device=dev), torch.zeros(8, rows, device=dev)
+        for i in range(0, nseq, step):
+            assert L.eva_k_flash_seq(P(q[i:]), P(k[i:]), P(v[i:]), P(o8[i * T_:]), P(s.reshape(-1)[i * T_:]), rows, step,
+                                     T_, TP, None, st) == 0
+        torch.cuda.synchronize()
+        return o8, s
+
+    for got, ref in zip(run(nseq), run(1)):
+        assert torch.equal(got, ref) and got.float().abs().sum() > 0
+
+
+@pytest.mark.parametrize("rows", [1, 15, 17, 5184 + 5])
+def test_hln_ragged_rows(dev, xt, orc, rows):
+    """rows that do not fill the last block of 16: y bit for bit, scores within the order of 32-bit sums, nothing
+    written past the last row"""
+    import numpy as np
+
+    print(f"px_k_hln: {rows} rows", flush=True)
+    r = np.random.default_rng(rows)
+    x = (r.standard_normal((rows, D)) * 1.5 + 0.2).astype(np.float16)
+    gw, gb = (1 + 0.1 * r.standard_normal(D)).astype(np.float32), (0.1 * r.standard_normal(D)).astype(np.float32)
+    hpos, U = (r.standard_normal((5184, D)) * 0.2).astype(np.float16), (r.standard_normal((16, D)) * 0.05).astype(np.float32)
+    d = [torch.from_numpy(a).to(dev) for a in (x, gw, gb, hpos, U)]
+    y, s = torch.full((rows + 16, D), 7, dtype=torch.int16, device=dev), torch.full((rows + 16, 16), 7.0, device=dev)
+    P = xt.ptr
+    assert xt.lib.px_k_hln(P(d[0]), P(d[1]), P(d[2]), P(d[3]), 5184, P(d[4]), P(y), P(s), rows,
+                           torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    y_ref, s_ref = orc.px_hln(x.view(np.uint16), 5184, gw, gb, hpos.view(np.uint16), U)
+    y, s = y.cpu().numpy(), s.cpu().numpy()
+    assert (y[:rows].view(np.uint16) == y_ref).all() and (y[rows:] == 7).all() and (s[rows:] == 7).all()
+    terms = np.abs(y_ref.view(np.float16).astype(np.float64)) @ np.abs(U.astype(np.float64)).T
+    assert np.all(np.abs(s[:rows] - s_ref) <= 2e-6 * terms)   # 32-bit sums of 1024 terms in two orders
