@@ -163,3 +163,56 @@ def test_hln_ragged_rows(dev, xt, orc, rows):
     assert (y[:rows].view(np.uint16) == y_ref).all() and (y[rows:] == 7).all() and (s[rows:] == 7).all()
     terms = np.abs(y_ref.view(np.float16).astype(np.float64)) @ np.abs(U.astype(np.float64)).T
     assert np.all(np.abs(s[:rows] - s_ref) <= 2e-6 * terms)   # 32-bit sums of 1024 terms in two orders
+
+
+@pytest.mark.parametrize("sparse", [False, True])
+@pytest.mark.parametrize("M,N,K,off,pad", [(1, 64, 128, 0, 0), (65, 207, 256, 1, 3), (1025, 3071, 1024, 0, 1),
+                                            (1025, 1024, 512, 3, 0), (2050, 3088, 128, 0, 0), (4100, 3072, 256, 5, 2),
+                                            (8200, 2000, 128, 0, 8), (1025, 13461, 128, 0, 0)])
+def test_gemm_any_alignment_and_tile(dev, xt, M, N, K, off, pad, sparse):
+    """C at any element offset and row stride, N ragged: the same bits as the fp32 output of the aligned call row by
+    row (in pieces of 64 rows: the smallest tiles), bf16 rounded to nearest even, nothing written outside C."""
+    N = (N + 15) // 16 * 16 if sparse else N
+    print(f"gemm {M} x {N} x {K}, offset {off}, pad {pad}, sparse {sparse}", flush=True)
+    L, P, st = xt.lib, xt.ptr, torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=dev)
+    g.manual_seed(M + N)
+    Np = (N + 127) // 128 * 128
+    a, sa = _codes(g, dev, M, K), torch.rand(K // 128, M + 64, generator=g, device=dev) * 0.01
+    w = _W(g, dev, Np, K, sparse)
+    fn = L.eva_k_gemm_sp if sparse else L.eva_k_gemm
+    ref = torch.zeros(M, Np, device=dev)
+    for r in range(0, M, 64):
+        assert fn(P(a[r:]), K, P(sa.reshape(-1)[r:]), M + 64, *w.args(xt), min(64, M - r), N, K, P(ref[r:]), Np, 1, st) == 0
+    for kind, dt in ((1, torch.float32), (0, torch.bfloat16)):
+        ldc = N + pad
+        buf = torch.full((off + M * ldc + 64,), 7.0, dtype=dt, device=dev)
+        assert fn(P(a), K, P(sa), M + 64, *w.args(xt), M, N, K, P(buf[off:]), ldc, kind, st) == 0
+        torch.cuda.synchronize()
+        want = torch.full_like(buf, 7.0)
+        want[off:off + M * ldc].view(M, ldc)[:, :N] = ref[:, :N].to(dt)
+        assert torch.equal(buf, want)
+
+
+@pytest.mark.parametrize("with_rs", [False, True])
+@pytest.mark.parametrize("rows", [12288, 12289])
+def test_px_fc1_rows_do_not_depend_on_the_tile(dev, xt, rows, with_rs):
+    print(f"px fc1: {rows} rows, rs {with_rs}", flush=True)
+    L, P, st = xt.lib, xt.ptr, torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=dev)
+    g.manual_seed(rows)
+    lds = rows + 256
+    h8, hs = _codes(g, dev, rows, D), torch.rand(8, lds, generator=g, device=dev) * 0.01
+    w, bias = _W(g, dev, PXH, D, False), torch.randn(PXH, generator=g, device=dev)
+    rs = torch.rand(PXH, generator=g, device=dev) + 0.5 if with_rs else None
+
+    def run(step):
+        m8, ms = torch.zeros(rows, PXH, dtype=U8, device=dev), torch.zeros(37, lds, device=dev)
+        for r in range(0, rows, step):
+            assert L.px_k_fc1(P(h8[r:]), P(hs.reshape(-1)[r:]), lds, *w.args(xt), P(bias), P(rs), P(m8[r:]),
+                              P(ms.reshape(-1)[r:]), min(step, rows - r), st) == 0
+        torch.cuda.synchronize()
+        return m8, ms
+
+    for got, ref in zip(run(rows), run(1000)):
+        assert torch.equal(got, ref)

@@ -428,8 +428,6 @@ __global__ void __launch_bounds__(256) k_head(const uint8_t *__restrict__ pq, co
 // PX: the PixAI patch GEMM (px_kernels.cu:133-138 k_ppe) instead: x[m] = f16(in[m] . pe^T) for window-major token rows
 // m (no cls, no position: k_px_pembed adds it before its LayerNorm), rows a multiple of 128.
 // ---------------------------------------------------------------------------------------------------------------
-typedef float v4f_e __attribute__((ext_vector_type(4), aligned(4)));     // 16 bytes of a buffer aligned to its
-typedef unsigned v4u_e __attribute__((ext_vector_type(4), aligned(2)));  // elements only (pos fp32, x fp16)
 template <class C, bool PX>
 __global__ void __launch_bounds__(C::NT) k_pe(const uint16_t *__restrict__ in, const uint16_t *__restrict__ pe,
                                               const float *__restrict__ pos, uint16_t *__restrict__ x, int rows)

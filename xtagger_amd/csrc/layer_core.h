@@ -69,6 +69,8 @@ __device__ __forceinline__ void layer_tile(int M, int N, int &m0, int &n0)
 }
 
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
+typedef float v4f_e __attribute__((ext_vector_type(4), aligned(4)));     // 16 bytes of memory aligned to its elements
+typedef unsigned v4u_e __attribute__((ext_vector_type(4), aligned(2)));  // only (fp32; 16-bit types)
 
 // x + y for the fp16 x in the low (HI = 0) or high (HI = 1) half of a word and an fp32 y: one v_fma_mix_f32,
 // fma(x, 1, y) with x widened exactly, which rounds once to fp32 as the conversion followed by v_add_f32 does

@@ -1,8 +1,7 @@
 // quant.hip - E4M3 packing with per-block fp32 scales (activations 1x128, weights 128x128) and the standalone
 // block-scaled GEMM. Reference roles: q2 / st4 / st8h (src/engine/kern_common.cuh:97-128) for activations,
 // fp8() (src/tools/export_eva.py:64-66) for weights, gemm8 (kern_common.cuh:271-356) for the GEMM.
-#include "gemm_core.h"
-#include "xt_abi.h"
+#include "layer_core.h"
 
 // ---- activations: x [M][ldx] (bf16, fp32 or fp16) -> q [M][ldq] E4M3, s [K/128][lds] ----
 // One thread per 8 consecutive elements; the 16 threads of one 128-element block are 16 aligned lanes.
@@ -112,20 +111,11 @@ __global__ void __launch_bounds__(256) k_scale_bits(uint32_t first, uint32_t cou
 }
 
 // ---- standalone block-scaled GEMM: C [M][ldc] = bf16 or fp32 of the block-scaled product ----
-// bf16: each wave parks 64 x 64 fp32 of its tile in its own LDS slice (row stride 68 floats, conflict-free), then
-// every lane rounds 8 consecutive columns to bf16 (RNE) and writes them with one 16-byte store through a descriptor
-// that ends at row M (rows past it are dropped). ldc and N multiples of 8 and a 16-byte aligned C take that path; other
-// shapes store element by element. fp32 (the parity build) stores straight from the accumulators.
-constexpr int GEMM_SLICE = 64 * 68 * 4;
-template <class C>
-constexpr int gemm_smem()
-{
-    return C::LDS > C::NW * GEMM_SLICE ? (C::LDS > C::LDS_SP ? C::LDS : C::LDS_SP)
-                                       : (C::NW * GEMM_SLICE > C::LDS_SP ? C::NW * GEMM_SLICE : C::LDS_SP);
-}
-
-typedef unsigned v4u __attribute__((ext_vector_type(4)));
-
+// bf16: each wave parks its rows x 64 (or 32) fp32 of its tile in its own LDS slice (padded rows, conflict-free), then
+// every lane rounds 8 consecutive columns to bf16 (RNE) and writes them with one 16-byte store, whatever the row's
+// alignment (the hardware takes 16-byte stores at any element address; two-byte stores for an odd ldc or N, as before,
+// took 242 us for 8200 x 13461 x 1024). fp32 stores 16 bytes straight from the accumulators. Columns of a store that
+// reaches past N go one by one.
 // SP: W holds the 2:4 values and WX the indices of the pack24 layout (bs_mainloop_sp); otherwise W is dense, WX unused.
 template <class C, int OUT, bool SP>  // OUT 0: bf16, 1: fp32
 __global__ void __launch_bounds__(C::NT) k_gemm(const uint8_t *__restrict__ A, int lda, const float *__restrict__ sa,
@@ -133,8 +123,7 @@ __global__ void __launch_bounds__(C::NT) k_gemm(const uint8_t *__restrict__ A, i
                                                const float *__restrict__ sw, void *__restrict__ Cp, int ldc, int M,
                                                int N, int K)
 {
-    static_assert(C::TM == 4 && C::TN % 4 == 0, "64-row wave tiles, whole 64-column passes");
-    __shared__ __attribute__((aligned(16))) uint8_t smem[gemm_smem<C>()];
+    __shared__ __attribute__((aligned(16))) uint8_t smem[LayerMem<C>::ROWSTAT];
     v4f acc[C::TM][C::TN];
     int tm, tn;
     tile_of_block((M + C::BM - 1) / C::BM, (N + C::BN - 1) / C::BN, M % C::BM != 0, tm, tn);
@@ -151,12 +140,11 @@ __global__ void __launch_bounds__(C::NT) k_gemm(const uint8_t *__restrict__ A, i
 #pragma unroll
             for (int j = 0; j < C::TN; j++) acc[i][j] = accT[j][i];
     } else {
-        bs_mainloop<C, BsNoPre, false, true>(A, lda, sa, lds, W, sw, M, Npad, K, m0, n0, smem, acc);
+        bs_mainloop<C, BsNoPre, C::TM == 2, true>(A, lda, sa, lds, W, sw, M, Npad, K, m0, n0, smem, acc);
     }
     int wm0, wn0;
     bs_wave_origin<C>(wm0, wn0);
-    if (OUT == 1) {
-        const bool v4ok = (ldc | N) % 4 == 0 && (((uintptr_t)Cp) & 15) == 0;  // whole 16-byte column quads
+    if constexpr (OUT == 1) {
 #pragma unroll
         for (int i = 0; i < C::TM; i++) {
             const int row = m0 + wm0 + 16 * i + c16;
@@ -165,8 +153,8 @@ __global__ void __launch_bounds__(C::NT) k_gemm(const uint8_t *__restrict__ A, i
 #pragma unroll
             for (int j = 0; j < C::TN; j++) {
                 const int col = n0 + wn0 + 16 * j + 4 * g;
-                if (v4ok) {
-                    if (col < N) *(float4 *)(crow + col) = make_float4(acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]);
+                if (col + 4 <= N) {
+                    *(v4f_e *)(crow + col) = acc[i][j];
                 } else {
 #pragma unroll
                     for (int r = 0; r < 4; r++)
@@ -174,52 +162,59 @@ __global__ void __launch_bounds__(C::NT) k_gemm(const uint8_t *__restrict__ A, i
                 }
             }
         }
-        return;
-    }
-    uint16_t *Cb = (uint16_t *)Cp;
-    if ((ldc | N) % 8 != 0 || (((uintptr_t)Cp) & 15)) {  // general shapes: one element per store
+    } else {
+        using S = LayerMem<C>;
+        constexpr int LPR = S::PC / 8, RPI = 64 / LPR;  // lanes a row, rows a store
+        float *tr = (float *)(smem + (threadIdx.x >> 6) * S::SLICE);
+        const int rs = lane / LPR, ch = lane % LPR;
 #pragma unroll
-        for (int i = 0; i < C::TM; i++)
+        for (int pass = 0; pass < C::WN / S::PC; pass++) {
+            if (pass) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the previous pass's slice reads are done
 #pragma unroll
-            for (int j = 0; j < C::TN; j++) {
-                const int row = m0 + wm0 + 16 * i + c16;
+            for (int i = 0; i < C::TM; i++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int col = n0 + wn0 + 16 * j + 4 * g + r;
-                    if (row < M && col < N) Cb[(size_t)row * ldc + col] = f2bf(acc[i][j][r]);
+                for (int j = 0; j < S::PC / 16; j++) {
+                    const v4f v = acc[i][S::PC / 16 * pass + j];
+                    *(float4 *)(tr + (16 * i + c16) * S::LD + 16 * j + 4 * g) = make_float4(v[0], v[1], v[2], v[3]);
+                }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slice is the wave's own: no block barrier needed
+            const int col = n0 + wn0 + S::PC * pass + 8 * ch;
+#pragma unroll
+            for (int it = 0; it < C::WM / RPI; it++) {
+                const int rr = RPI * it + rs, row = m0 + wm0 + rr;
+                const float *t = tr + rr * S::LD + 8 * ch;
+                const float4 a = *(const float4 *)t, b = *(const float4 *)(t + 4);
+                uint16_t *c = (uint16_t *)Cp + (size_t)row * ldc + col;
+                if (row < M && col + 8 <= N) {
+                    *(v4u_e *)c = v4u_e{f2bf(a.x) | (uint32_t)f2bf(a.y) << 16, f2bf(a.z) | (uint32_t)f2bf(a.w) << 16,
+                                        f2bf(b.x) | (uint32_t)f2bf(b.y) << 16, f2bf(b.z) | (uint32_t)f2bf(b.w) << 16};
+                } else if (row < M) {
+                    for (int e = 0; col + e < N; e++) c[e] = f2bf(t[e]);
                 }
             }
-        return;
-    }
-    float *tr = (float *)(smem + (threadIdx.x >> 6) * GEMM_SLICE);
-    const __amdgpu_buffer_rsrc_t rc = buf_rsrc(Cp, (uint32_t)M * (uint32_t)ldc * 2u);
-    const int rs = lane >> 3, ch = lane & 7;
-#pragma unroll
-    for (int pass = 0; pass < C::TN / 4; pass++) {
-        if (pass) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the previous pass's slice reads are done
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const v4f v = acc[i][4 * pass + j];
-                *(float4 *)(tr + (16 * i + c16) * 68 + 16 * j + 4 * g) = make_float4(v[0], v[1], v[2], v[3]);
-            }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slice is the wave's own: no block barrier needed
-        const int col = n0 + wn0 + 64 * pass + 8 * ch;
-#pragma unroll
-        for (int it = 0; it < 8; it++) {
-            const int rr = 8 * it + rs;
-            const float4 a = *(const float4 *)(tr + rr * 68 + 8 * ch), b = *(const float4 *)(tr + rr * 68 + 8 * ch + 4);
-            const v4u o = {f2bf(a.x) | (uint32_t)f2bf(a.y) << 16, f2bf(a.z) | (uint32_t)f2bf(a.w) << 16,
-                           f2bf(b.x) | (uint32_t)f2bf(b.y) << 16, f2bf(b.z) | (uint32_t)f2bf(b.w) << 16};
-            if (col < N)
-                __builtin_amdgcn_raw_buffer_store_b128(o, rc, (int)(((uint32_t)(m0 + wm0 + rr) * (uint32_t)ldc + col) * 2u), 0, 0);
         }
     }
 }
 
-typedef BsCfg<256, 256, 4, 2, 2> GemmBig;    // 8 waves of 64 x 128, 2 stages: once the tiles fill the 256 CUs
-typedef BsCfg<128, 128, 2, 2, 2> GemmMid;    // 4 waves of 64 x 64, 2 stages, two blocks per CU: small M
+// Tiles by how many there are (us; bf16 output, dense unless said):
+//  - 64 x 64 while one round of two blocks per CU holds them: 128 x 128 -> 64 x 64 at 1 x 1000 x 4736 (M x N x K) 22.5 ->
+//    12.0, 100 x 13461 x 1024 10.9 -> 7.3, 1025 x 1024 x 1024 7.8 -> 6.1 (64 x 128: 16.5, 8.7, 6.6);
+//  - 64 x 128 likewise: 1025 x 3072 x 1024 9.05 -> 8.7, x 4736 31.9 -> 25.1 (64 x 64: 10.4, 32.2);
+//  - 256 x 256 where they fill one round, or 1.6 and more (2:4-sparse 4322 x 6256 x 4608 116.7 against 121.4): 4100 x
+//    3072 x 1024 19.8 against 21.6 for 128 x 128, 2:4-sparse 8200 x 13456 x 1024 138 against 146;
+//  - 128 x 128 elsewhere: 2050 x 3072 x 1024 18.1 -> 12.6, 1025 x 13461 x 1024 51.1 -> 39.5, 4100 x 5000 x 2048 61.2 ->
+//    55.6 (the tile before was 256 x 256 from 256 of them on).
+typedef BsCfg<64, 64, 2, 2, 3> GemmSml;
+template <class F>
+static void with_gemm_cfg(int M, int N, F f)
+{
+    auto tiles = [&](auto c) { return (long)((M + c.BM - 1) / c.BM) * ((N + c.BN - 1) / c.BN); };
+    const long big = tiles(LayerCfg{});
+    if (tiles(GemmSml{}) <= 512) f(GemmSml{});
+    else if (tiles(LayerSml{}) <= 512) f(LayerSml{});
+    else if ((big >= 192 && big <= 256) || big >= 410) f(LayerCfg{});
+    else f(LayerMid{});
+}
 
 // ---------------------------------------------------------------------------------------------------------------
 // C-ABI launchers
@@ -297,25 +292,14 @@ static int gemm_launch(const char *what, const void *qa, int lda, const float *s
     const uint8_t *A = (const uint8_t *)qa, *W = (const uint8_t *)qw;
     const uint32_t *X = (const uint32_t *)qx;
     hipStream_t st = (hipStream_t)stream;
-    // big tiles once there are enough of them to fill the 256 CUs, else 128 x 128 tiles (two blocks per CU)
-    const long big = (long)((M + GemmBig::BM - 1) / GemmBig::BM) * ((N + GemmBig::BN - 1) / GemmBig::BN);
-    if (big >= 256) {
-        const dim3 grid((unsigned)big);
+    with_gemm_cfg(M, N, [&](auto c_) {
+        using T = decltype(c_);
+        const dim3 grid((unsigned)(((M + T::BM - 1) / T::BM) * ((N + T::BN - 1) / T::BN)));
         if (out_kind == 0)
-            hipLaunchKernelGGL((k_gemm<GemmBig, 0, SP>), grid, dim3(GemmBig::NT), 0, st, A, lda, sa, lds, W, X, sw, c,
-                               ldc, M, N, K);
+            hipLaunchKernelGGL((k_gemm<T, 0, SP>), grid, dim3(T::NT), 0, st, A, lda, sa, lds, W, X, sw, c, ldc, M, N, K);
         else
-            hipLaunchKernelGGL((k_gemm<GemmBig, 1, SP>), grid, dim3(GemmBig::NT), 0, st, A, lda, sa, lds, W, X, sw, c,
-                               ldc, M, N, K);
-    } else {
-        const dim3 grid((unsigned)(((M + GemmMid::BM - 1) / GemmMid::BM) * ((N + GemmMid::BN - 1) / GemmMid::BN)));
-        if (out_kind == 0)
-            hipLaunchKernelGGL((k_gemm<GemmMid, 0, SP>), grid, dim3(GemmMid::NT), 0, st, A, lda, sa, lds, W, X, sw, c,
-                               ldc, M, N, K);
-        else
-            hipLaunchKernelGGL((k_gemm<GemmMid, 1, SP>), grid, dim3(GemmMid::NT), 0, st, A, lda, sa, lds, W, X, sw, c,
-                               ldc, M, N, K);
-    }
+            hipLaunchKernelGGL((k_gemm<T, 1, SP>), grid, dim3(T::NT), 0, st, A, lda, sa, lds, W, X, sw, c, ldc, M, N, K);
+    });
     return xt_check(what);
 }
 
