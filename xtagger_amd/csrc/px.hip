@@ -164,16 +164,15 @@ __global__ void __launch_bounds__(C::NT) k_px_res(const uint8_t *__restrict__ a8
 // bytes per lane (8 rows of 64 bytes per wave instruction). The second half of the last column tile lies past
 // unit 4736 and stores nothing.
 // ---------------------------------------------------------------------------------------------------------------
-template <bool SP, bool RS>
-__global__ void __launch_bounds__(LayerCfg::NT) k_px_fc1(const uint8_t *__restrict__ h8, const float *__restrict__ hs,
-                                                        int lds, const uint8_t *__restrict__ w,
-                                                        const uint32_t *__restrict__ wx, const float *__restrict__ ws,
+template <class C, bool RS>
+__global__ void __launch_bounds__(C::NT) k_px_fc1(const uint8_t *__restrict__ h8, const float *__restrict__ hs,
+                                                        int lds, const uint8_t *__restrict__ w, const float *__restrict__ ws,
                                                         const float *__restrict__ bias, const float *__restrict__ rs,
                                                         uint8_t *__restrict__ m8, float *__restrict__ ms, int rows)
 {
-    using C = LayerCfg;
-    static_assert(C::TM == 4 && C::TN == 8 && C::WN == 128, "a wave tile is 64 rows x one 128-unit scale block");
-    __shared__ __attribute__((aligned(16))) uint8_t smem[LayerMem<C>::SMEM];
+    using S = LayerMem<C>;
+    static_assert(C::WN == 128, "a wave's columns are one 128-unit scale block");
+    __shared__ __attribute__((aligned(16))) uint8_t smem[S::ROWSTAT];
     v4f acc[C::TM][C::TN];
     int m0, n0, wm0, wn0;
     layer_tile<C>(rows, PX_HID, m0, n0);
@@ -181,7 +180,7 @@ __global__ void __launch_bounds__(LayerCfg::NT) k_px_fc1(const uint8_t *__restri
     // the tile transposed (TR): lane (g, c16) holds row m0 + wm0 + 16 i + c16 and units 128 blk + 16 j + 4 g + r, so
     // a row's 128 units lie in the 4 lanes that share c16: its |max| meets in two lane swaps, one scale per lane and
     // row tile
-    layer_mainloop<C, SP, BsNoPre, true>(h8, XT_D, hs, lds, w, wx, ws, rows, PX_HID, XT_D, m0, n0, smem, acc);
+    layer_mainloop<C, false, BsNoPre, true>(h8, XT_D, hs, lds, w, nullptr, ws, rows, PX_HID, XT_D, m0, n0, smem, acc);
     bs_wave_origin<C>(wm0, wn0);
     const int blk = (n0 + wn0) >> 7;
     if (blk >= PX_HID / 128) return;  // no block barrier follows: the epilogue uses the wave's own slice only
@@ -213,7 +212,7 @@ __global__ void __launch_bounds__(LayerCfg::NT) k_px_fc1(const uint8_t *__restri
         const int m = m0 + wm0 + 16 * i + c16;
         if (g == 0 && m < rows) ms[(size_t)blk * lds + m] = sc;
     }
-    float *tr = (float *)(smem + (threadIdx.x >> 6) * LayerMem<C>::SLICE);
+    float *tr = (float *)(smem + (threadIdx.x >> 6) * S::SLICE);
     const __amdgpu_buffer_rsrc_t rm = buf_rsrc(m8, (uint32_t)rows * PX_HID);
     const int rsub = lane >> 3, ch = lane & 7;
 #pragma unroll
@@ -229,7 +228,7 @@ __global__ void __launch_bounds__(LayerCfg::NT) k_px_fc1(const uint8_t *__restri
             }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slice is the wave's own: no block barrier needed
 #pragma unroll
-        for (int it = 0; it < 8; it++) {
+        for (int it = 0; it < C::WM / 8; it++) {
             const int rr = 8 * it + rsub;
             const float4 a = *(const float4 *)(tr + rr * 68 + 8 * ch), b = *(const float4 *)(tr + rr * 68 + 8 * ch + 4);
             typedef unsigned v2u __attribute__((ext_vector_type(2)));
@@ -283,16 +282,33 @@ extern "C" int px_k_fc2(const void *m8, const float *ms, int lds, const void *w,
     return px_res_launch<PX_HID>("px_k_fc2", m8, ms, lds, w, ws, bias, x, rows, stream);
 }
 
+// k_px_fc1's tiles: 128 x 128 (4 waves of 32 x 128, two blocks per CU) up to 12288 rows: one block's GELU and packing
+// runs beside the other's main loop, and the last round wastes less (48.0 -> 41.4 us at 5184 rows, 85.2 -> 77.0 at
+// 10368); with more rounds 256 x 256 is as good or better (111 against 114 at 15552, 290 against 292 at 41472).
+typedef BsCfg<128, 128, 4, 1, 2> PxFc1Mid;
+template <class F>
+static void with_px_fc1_cfg(int rows, F f)
+{
+    if (rows <= 12288) f(PxFc1Mid{});
+    else f(LayerCfg{});
+}
+
 extern "C" int px_k_fc1(const void *h8, const float *hs, int lds, const void *w, const float *ws, const float *bias,
                         const float *rs, void *m8, float *ms, int rows, void *stream)
 {
     if (layer_rows_ok("px_k_fc1", rows, lds)) return -1;
     if (!XT_ALIGNED(h8) || !XT_ALIGNED(w) || ((uintptr_t)m8 & 7))
         return xt_fail("px_k_fc1", "h8 and w must be 16-byte aligned, m8 8-byte aligned");
-    auto kern = rs ? k_px_fc1<false, true> : k_px_fc1<false, false>;  // the multiply only where rs is given
-    hipLaunchKernelGGL(kern, dim3(layer_grid<LayerCfg>(rows, PX_HID)), dim3(LayerCfg::NT), 0,
-                       (hipStream_t)stream, (const uint8_t *)h8, hs, lds, (const uint8_t *)w, (const uint32_t *)nullptr,
-                       ws, bias, rs, (uint8_t *)m8, ms, rows);
+    with_px_fc1_cfg(rows, [&](auto c) {
+        using C = decltype(c);
+        const dim3 grid(layer_grid<C>(rows, PX_HID));
+        if (rs)  // the multiply only where rs is given
+            hipLaunchKernelGGL((k_px_fc1<C, true>), grid, dim3(C::NT), 0, (hipStream_t)stream, (const uint8_t *)h8, hs,
+                               lds, (const uint8_t *)w, ws, bias, rs, (uint8_t *)m8, ms, rows);
+        else
+            hipLaunchKernelGGL((k_px_fc1<C, false>), grid, dim3(C::NT), 0, (hipStream_t)stream, (const uint8_t *)h8, hs,
+                               lds, (const uint8_t *)w, ws, bias, rs, (uint8_t *)m8, ms, rows);
+    });
     return xt_check("px_k_fc1");
 }
 
