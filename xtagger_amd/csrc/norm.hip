@@ -152,7 +152,7 @@ __global__ void __launch_bounds__(512) k_pool(const uint16_t *__restrict__ x, fl
     float s[8];
 #pragma unroll
     for (int k = 0; k < 8; k++) s[k] = 0.f;
-#pragma unroll 8
+#pragma unroll
     for (int t = 0; t < 32; t++) {
         const uint4 u = *(const uint4 *)(xr + (size_t)t * XT_D);
         const uint32_t w[4] = {u.x, u.y, u.z, u.w};
