@@ -234,20 +234,19 @@ size_t eva_img_pyramid_bytes(uint32_t w, uint32_t h, uint32_t S);
 /* pi_pyramid: levels 1.. of p into `levels` (32-byte aligned, eva_img_pyramid_bytes), 2x2 boxes of pi_half
  * (procimg.h:636-661); sets p->nlv and the level fields. */
 int eva_img_pyramid(eva_pyr *p, void *levels, size_t bytes, uint32_t S, void *stream);
-/* Scratch bytes of eva_img_prep for crops whose long side on the chosen level is at most max_side (4 S - 1 covers
+/* Scratch bytes that eva_img_prep asks for with crops whose long side on the chosen level is at most max_side (4 S - 1 covers
  * every crop of a full pyramid). */
 size_t eva_img_prep_bytes(uint32_t S, uint32_t max_side);
 /* pi_prep (procimg.h:926-969): the level-0 rect (x0, y0, cw, ch) -> out fp16 [(S/14)^2][592] (EVA_IN halves at
  * S = 448; 16-byte aligned), resampled (bicubic onto the white square, [-1, 1], BGR planes) from the level pi_level
- * picks, or normalised as is when the rect's long side on that level is S. The 4 pad halves of each patch row are 0. */
+ * picks, or normalised as is when the rect's long side on that level is S. The 4 pad halves of each patch row are 0.
+ * scratch and bytes are checked (16-byte aligned, S x rect width on the level x 16 bytes) and nothing is written there. */
 int eva_img_prep(const eva_pyr *p, uint32_t x0, uint32_t y0, uint32_t cw, uint32_t ch, uint32_t S, void *scratch,
                  size_t bytes, void *out, void *stream);
 /* eva_img_prep that allocates nothing and takes no scratch argument. No counterpart in the reference: it is for callers
- * that cannot allocate (code under HIP graph capture, tight serving loops). The vertical pass is staged in a
- * library-owned device array of EVA_IMG_STATIC_BYTES on each GPU it runs on (held until the process ends; its address
- * is looked up on the first call on each device): rects whose chosen level needs more than that (S x rect width on
- * the level x 16 bytes, i.e. the long side on the level below 4 S - 1 at S = 448) fail with -1. All calls on one GPU
- * share the array: calls that overlap in time on that GPU race, so issue them on one stream. */
+ * that cannot allocate (code under HIP graph capture, tight serving loops). Nothing is staged in memory, so calls on
+ * several streams may overlap; rects whose chosen level would need more scratch than EVA_IMG_STATIC_BYTES (S x rect
+ * width on the level x 16 bytes, i.e. the long side on the level below 4 S - 1 at S = 448) fail with -1. */
 #define EVA_IMG_STATIC_BYTES ((size_t)448 * (4 * 448 - 1) * 16)
 int eva_img_prep_static(const eva_pyr *p, uint32_t x0, uint32_t y0, uint32_t cw, uint32_t ch, uint32_t S, void *out,
                         void *stream);

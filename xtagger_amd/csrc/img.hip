@@ -7,35 +7,45 @@
 // one fma per tap in tap order (vertical pass, then horizontal pass over RGBX), clamp to [-1, 1], fp16 by
 // round-to-nearest-even. The outputs are therefore bit-identical to the reference's.
 //
-// Data flow of one crop (eva_img_prep): the host picks the level and the rect on it (pi_level / pi_lsrc, scalar), then
-//   k_img_vpass tmp [S][cw * 4] fp32: output row i over the rect's columns, all RGBX channels (pi_vrow);
-//   k_img_hpass one 14-row band of 2 patches per block: each output pixel's B, G, R over its horizontal taps (pi_hrow),
-//               staged in shared memory in the operand's own layout and written out as contiguous 16-byte stores.
-// Each block builds the tap tables it needs (pi_axis) in shared memory: every tap weight in parallel, each output's sum
-// over its taps in the reference's order by one thread.
+// One crop (eva_img_prep): the host picks the level and the rect on it (pi_level / pi_lsrc, scalar), then
+// k_img_resample takes one 14-row band of 2 patches per block: both axes' tap tables (pi_axis) in shared memory, the
+// vertical pass over the source columns the band takes (pi_vrow), the horizontal pass from there (pi_hrow), staged in
+// shared memory in the operand's own layout and written out as contiguous 16-byte stores.
 // A rect whose long side is S skips the resample (pi_idrow): k_img_ident normalises and white-pads the band directly.
-#include <pthread.h>
-
 #include "xt_abi.h"
 #include "xtag_eva.h"
 
 #define IMG_BAND_P 2                        // patches per band block (2 x 592 halves = 2368 contiguous bytes)
 #define IMG_PATCH 592                       // halves per patch row of the operand (588 + 4 zero pad)
 
-// ---- pi_row_rgbx with alpha (procimg.h:592-630): c -> (c a + 255 (255 - a)) / 255 rounded, X = 255, in place
-__global__ void __launch_bounds__(256) k_img_over_white(uint8_t *__restrict__ p, size_t stride, uint32_t w, uint32_t h)
+// ---- pi_row_rgbx with alpha (procimg.h:592-630): c -> (c a + 255 (255 - a)) / 255 rounded, X = 255, in place. Four
+// pixels a thread (16 bytes at any pixel's alignment; a row's last pixels one by one); opaque pixels are left as they
+// are by the formula ((255 c) / 255 = c, X = 255 already), so four of them are not written back. Bound by HBM: 3072 x
+// 2048 with a translucent corner 13.6 -> 6 us against a read and a write of four bytes per thread.
+typedef unsigned img_u4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ uint32_t img_white(uint32_t v)
 {
-    const uint32_t x = blockIdx.x * 256 + threadIdx.x, y = blockIdx.y;
-    if (x >= w || y >= h) return;
-    uint32_t *px = (uint32_t *)(p + (size_t)y * stride) + x;
-    const uint32_t v = *px, a = v >> 24, ia = 255u * (255u - a);
+    const uint32_t a = v >> 24, ia = 255u * (255u - a);
     uint32_t o = 0xFF000000u;
 #pragma unroll
     for (int c = 0; c < 3; c++) {
         const uint32_t t = ((v >> (8 * c)) & 255u) * a + ia;
         o |= ((t + 128u + ((t + 128u) >> 8)) >> 8) << (8 * c);
     }
-    *px = o;
+    return o;
+}
+__global__ void __launch_bounds__(256) k_img_over_white(uint8_t *__restrict__ p, size_t stride, uint32_t w, uint32_t h)
+{
+    const uint32_t x = 4 * (blockIdx.x * 64 + (threadIdx.x & 63)), y = blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (x >= w || y >= h) return;
+    uint32_t *px = (uint32_t *)(p + (size_t)y * stride) + x;
+    if (w - x < 4) {
+        for (uint32_t i = 0; i < w - x; i++) px[i] = img_white(px[i]);
+        return;
+    }
+    const img_u4 v = *(const img_u4 *)px;
+    if ((v[0] & v[1] & v[2] & v[3]) >> 24 == 255u) return;
+    *(img_u4 *)px = img_u4{img_white(v[0]), img_white(v[1]), img_white(v[2]), img_white(v[3])};
 }
 
 // ---- pi_half (procimg.h:636-661): one level of the 2x2 box pyramid, per output pixel and channel
@@ -101,72 +111,81 @@ __device__ __forceinline__ void img_bounds(const ImgGeom &g, int32_t i, float &c
     b = b < a ? a : b;
 }
 
-// Tap tables of `cnt` consecutive outputs i0 .. i0 + cnt - 1 into shared memory: every tap weight in parallel (the same
-// float expression as the reference), then one thread per output sums its taps in tap order (the reference's loop),
-// then the content taps are scaled. w [cnt][mt] holds the content taps; s, n, k per output. Ends synchronised.
-__device__ __forceinline__ void img_taps(const ImgGeom &g, int32_t i0, int32_t cnt, int32_t mt, float *w, int32_t *s,
-                                         int32_t *n, float *k, float *sum)
+#define IMG_MT_MAX 24                       // taps per output up to a resample factor of 5 (mt = 2 (int)(2 f + 1) + 2)
+#define IMG_XN (14 * IMG_BAND_P)            // outputs of a block's two axes: 28 columns, then 14 rows
+#define IMG_ON (IMG_XN + 14)
+#define IMG_RT 512                          // threads of k_img_resample
+#define IMG_SPAN 176                        // source columns of 28 outputs at that factor: 28 f + 4 f + 2 rounded up
+
+// Tap tables (shared memory) of a block's outputs: columns x0 .. x0 + nx - 1 as outputs 0 .., rows y0 .. y0 + 13 as
+// outputs IMG_XN ..: every raw weight in parallel (the same float expression as the reference), then one thread per
+// output sums its taps in tap order (the reference's loop; taps past the last add an exact zero, so the loop has a
+// fixed length and its reads overlap), then the content taps, scaled, in parallel again. w [output][mt] holds the
+// content taps; s, n, k per output. Ends synchronised.
+struct ImgTaps {
+    float raw[IMG_ON * IMG_MT_MAX], w[IMG_ON * IMG_MT_MAX], k[IMG_ON], sum[IMG_ON];
+    int32_t s[IMG_ON], n[IMG_ON], skip[IMG_ON];
+};
+
+// gy or gx, field by field (a reference to either would put both in scratch memory); the axes share the square
+__device__ __forceinline__ ImgGeom img_axis(const ImgGeom &gx, const ImgGeom &gy, bool y)
 {
-    for (int32_t e = threadIdx.x; e < cnt * mt; e += blockDim.x) {
-        const int32_t c = e / mt, t = e - c * mt;
-        float center;
-        int32_t lo, hi, a, b;
-        img_bounds(g, i0 + c, center, lo, hi, a, b);
-        w[e] = lo + t < hi ? img_cubic(((float)(lo + t) - center + 0.5f) * g.ss) : 0.0f;
-    }
-    __syncthreads();
-    for (int32_t c = threadIdx.x; c < cnt; c += blockDim.x) {
-        float center, sm = 0.0f, white = 0.0f;
-        int32_t lo, hi, a, b;
-        img_bounds(g, i0 + c, center, lo, hi, a, b);
-        for (int32_t j = lo; j < hi; j++) {
-            const float wt = w[c * mt + (j - lo)];
-            sm += wt;
-            white += j < a || j >= b ? wt : 0.0f;
-        }
-        sm = g.sc / sm;
-        sum[c] = sm;
-        s[c] = a - g.off;
-        n[c] = b - a;
-        k[c] = 255.0f * white * sm + g.add;
-    }
-    __syncthreads();
-    // content taps to the front of the row, scaled (pi_axis's memmove and wi[j] *= sum), in place: each thread moves
-    // the taps of one output so no row is read after another thread overwrote it
-    for (int32_t c = threadIdx.x; c < cnt; c += blockDim.x) {
-        float center;
-        int32_t lo, hi, a, b;
-        img_bounds(g, i0 + c, center, lo, hi, a, b);
-        for (int32_t q = 0; q < b - a; q++) w[c * mt + q] = w[c * mt + (a - lo) + q] * sum[c];
-    }
-    __syncthreads();
+    ImgGeom g = gx;
+    g.sc = y ? gy.sc : gx.sc;
+    g.add = y ? gy.add : gx.add;
+    g.off = y ? gy.off : gx.off;
+    g.end = y ? gy.end : gx.end;
+    return g;
 }
 
-#define IMG_MT_MAX 24                       // taps per output up to a resample factor of 5 (mt = 2 (int)(2 f + 1) + 2)
-
-// ---- pi_vrow (procimg.h:800-836): tmp[i][4 x + c] = k + sum_j w[j] * src(s + j)[x].c, one RGBX pixel per thread;
-// block (blockIdx.x, i = blockIdx.y) builds the y tap table of output row i
-__global__ void __launch_bounds__(256) k_img_vpass(const uint8_t *__restrict__ src, size_t stride, uint32_t cw,
-                                                   uint32_t ch, uint32_t S, uint32_t side, uint32_t mt,
-                                                   float4 *__restrict__ tmp)
+__device__ __forceinline__ void img_taps(const ImgGeom &gx, const ImgGeom &gy, int32_t x0, int32_t nx, int32_t y0,
+                                         int32_t mt, ImgTaps &T)
 {
-    __shared__ float w[IMG_MT_MAX], sum[1], k[1];
-    __shared__ int32_t sn[2];
-    const uint32_t i = blockIdx.y, x = blockIdx.x * 256 + threadIdx.x;
-    img_taps(img_geom(S, side, (side - ch) >> 1, ch, 1.0f, 0.0f), (int32_t)i, 1, (int32_t)mt, w, sn, sn + 1, k, sum);
-    if (x >= cw) return;
-    const int32_t s = sn[0], n = sn[1];
-    float a0 = k[0], a1 = a0, a2 = a0, a3 = a0;
-    const uint8_t *p = src + (size_t)s * stride + 4 * (size_t)x;
-    for (int32_t j = 0; j < n; j++, p += stride) {
-        const uint32_t v = *(const uint32_t *)p;
-        const float wj = w[j];
-        a0 = __builtin_fmaf(wj, (float)(v & 255u), a0);
-        a1 = __builtin_fmaf(wj, (float)((v >> 8) & 255u), a1);
-        a2 = __builtin_fmaf(wj, (float)((v >> 16) & 255u), a2);
-        a3 = __builtin_fmaf(wj, (float)(v >> 24), a3);
+    for (int32_t e = threadIdx.x; e < IMG_ON * IMG_MT_MAX; e += blockDim.x) {
+        const int32_t c = e / IMG_MT_MAX, t = e - c * IMG_MT_MAX;
+        const bool y = c >= IMG_XN;
+        float wt = 0.0f;
+        if (t < mt && (y || c < nx)) {
+            const ImgGeom g = img_axis(gx, gy, y);
+            float center;
+            int32_t lo, hi, a, b;
+            img_bounds(g, y ? y0 + c - IMG_XN : x0 + c, center, lo, hi, a, b);
+            wt = lo + t < hi ? img_cubic(((float)(lo + t) - center + 0.5f) * g.ss) : 0.0f;
+        }
+        T.raw[e] = wt;
     }
-    tmp[(size_t)i * cw + x] = make_float4(a0, a1, a2, a3);
+    __syncthreads();
+    if (threadIdx.x < IMG_ON) {
+        const int32_t c = threadIdx.x;
+        const bool y = c >= IMG_XN;
+        if (y || c < nx) {
+            const ImgGeom g = img_axis(gx, gy, y);
+            float center, sm = 0.0f, white = 0.0f;
+            int32_t lo, hi, a, b;
+            img_bounds(g, y ? y0 + c - IMG_XN : x0 + c, center, lo, hi, a, b);
+#pragma unroll
+            for (int32_t t = 0; t < IMG_MT_MAX; t++) {
+                const float wt = T.raw[c * IMG_MT_MAX + t];
+                sm += wt;
+                white += lo + t < a || lo + t >= b ? wt : 0.0f;
+            }
+            sm = g.sc / sm;
+            T.sum[c] = sm;
+            T.s[c] = a - g.off;
+            T.n[c] = b - a;
+            T.skip[c] = a - lo;
+            T.k[c] = 255.0f * white * sm + g.add;
+        } else {
+            T.s[c] = T.n[c] = T.skip[c] = 0;
+            T.sum[c] = T.k[c] = 0.0f;
+        }
+    }
+    __syncthreads();
+    for (int32_t e = threadIdx.x; e < IMG_ON * IMG_MT_MAX; e += blockDim.x) {
+        const int32_t c = e / IMG_MT_MAX, t = e - c * IMG_MT_MAX;
+        T.w[e] = t < T.n[c] ? T.raw[e + T.skip[c]] * T.sum[c] : 0.0f;  // skip + n <= mt
+    }
+    __syncthreads();
 }
 
 __device__ __forceinline__ uint16_t img_f16(float v)
@@ -185,34 +204,71 @@ __device__ __forceinline__ void img_band_store(uint16_t *band, uint16_t *__restr
     for (uint32_t q = threadIdx.x; q < np * IMG_PATCH / 8; q += blockDim.x) dst[q] = sb[q];
 }
 
-// ---- pi_hrow (procimg.h:843-868): band blockIdx.y, patches blockIdx.x * IMG_BAND_P ..; one output pixel per
-// thread; the block builds the x tap tables of its 14 IMG_BAND_P columns
-__global__ void __launch_bounds__(14 * 14 * IMG_BAND_P) k_img_hpass(const float4 *__restrict__ tmp, uint32_t cw,
-                                                                  uint32_t S, uint32_t side, uint32_t mt,
-                                                                  uint16_t *__restrict__ out)
+// ---- pi_vrow and pi_hrow (procimg.h:800-868) of one band: rows 14 blockIdx.y .., patches blockIdx.x * IMG_BAND_P ..
+// The block resamples vertically only the source columns its 28 output columns take (14 rows x those columns, RGB in
+// fp32, into shared memory: neighbouring blocks repeat the taps' overlap, about a seventh), then horizontally from
+// there, one output pixel per thread. Each value is the constant plus one fma per tap in tap order, as in the
+// reference's two passes over whole rows. Bound by the latency of its steps (tap tables, source reads, horizontal taps)
+// at these sizes; 512 threads a block (392: 10% slower, 832: 40%). us a call, two kernels with the vertical result in
+// an fp32 [S][cw] scratch in between -> here: 3072 x 2048 at level 1 17.6 -> 13.1, 1847 x 2048 13.4 -> 11.1, 900 x 900
+// at level 0 12.4 -> 9.7, 440 x 300 8.9 -> 7.4.
+__global__ void __launch_bounds__(IMG_RT) k_img_resample(const uint8_t *__restrict__ src, size_t stride,
+                                                                     uint32_t cw, uint32_t ch, uint32_t S,
+                                                                     uint32_t side, uint32_t mt,
+                                                                     uint16_t *__restrict__ out)
 {
     __shared__ __attribute__((aligned(16))) uint16_t band[IMG_BAND_P * IMG_PATCH];
-    __shared__ float w[14 * IMG_BAND_P * IMG_MT_MAX], k[14 * IMG_BAND_P], sum[14 * IMG_BAND_P];
-    __shared__ int32_t ts[14 * IMG_BAND_P], tn[14 * IMG_BAND_P];
+    __shared__ ImgTaps T;
+    __shared__ float v[3][14 * IMG_SPAN];
+    __shared__ int32_t span[2];
     const uint32_t pr = S / 14, pc0 = blockIdx.x * IMG_BAND_P;
     const uint32_t np = pr - pc0 < IMG_BAND_P ? pr - pc0 : IMG_BAND_P;
+    const int32_t nx = (int32_t)(14 * np);
     if (threadIdx.x < np) *(uint2 *)(band + threadIdx.x * IMG_PATCH + 588) = uint2{0u, 0u};
-    img_taps(img_geom(S, side, (side - cw) >> 1, cw, 1.0f / 127.5f, -1.0f), (int32_t)(pc0 * 14), (int32_t)(14 * np),
-             (int32_t)mt, w, ts, tn, k, sum);
+    if (threadIdx.x == 0) span[0] = 0x7fffffff, span[1] = 0;
+    img_taps(img_geom(S, side, (side - cw) >> 1, cw, 1.0f / 127.5f, -1.0f), img_geom(S, side, (side - ch) >> 1, ch, 1.0f, 0.0f),
+             (int32_t)(pc0 * 14), nx, (int32_t)(blockIdx.y * 14), (int32_t)mt, T);
+    if (threadIdx.x < IMG_XN && T.n[threadIdx.x]) {  // source columns [span[0], span[1]) that any output takes
+        atomicMin(&span[0], T.s[threadIdx.x]);
+        atomicMax(&span[1], T.s[threadIdx.x] + T.n[threadIdx.x]);
+    }
+    __syncthreads();
+    const int32_t x0 = span[0], nc = span[1] - x0, nw = nc < 0 ? 0 : nc < IMG_SPAN ? nc : IMG_SPAN;
+    for (int32_t e = threadIdx.x; e < 14 * nw; e += blockDim.x) {
+        const int32_t ky = e / nw, x = e - ky * nw, c = IMG_XN + ky, n = T.n[c];
+        const float *wj = T.w + c * IMG_MT_MAX;
+        float a0 = T.k[c], a1 = a0, a2 = a0;
+        const uint8_t *p = src + (size_t)T.s[c] * stride + 4 * (size_t)(x0 + x);
+        // eight source pixels in flight; past the last tap its row again, with weight 0 (adds an exact zero)
+        for (int32_t j0 = 0; j0 < n; j0 += 8) {
+            uint32_t u[8];
+#pragma unroll
+            for (int32_t j = 0; j < 8; j++) u[j] = *(const uint32_t *)(p + (size_t)(j0 + j < n ? j0 + j : n - 1) * stride);
+#pragma unroll
+            for (int32_t j = 0; j < 8; j++) {
+                const float w = wj[j0 + j];
+                a0 = __builtin_fmaf(w, (float)(u[j] & 255u), a0);
+                a1 = __builtin_fmaf(w, (float)((u[j] >> 8) & 255u), a1);
+                a2 = __builtin_fmaf(w, (float)((u[j] >> 16) & 255u), a2);
+            }
+        }
+        v[0][ky * IMG_SPAN + x] = a0;
+        v[1][ky * IMG_SPAN + x] = a1;
+        v[2][ky * IMG_SPAN + x] = a2;
+    }
+    __syncthreads();
     const uint32_t e = threadIdx.x;
     if (e < 14 * 14 * np) {
         const uint32_t ky = e / (14 * np), jj = e - ky * 14 * np;   // row in the band, column in the block
-        const uint32_t i = blockIdx.y * 14 + ky;
-        const int32_t n = tn[jj];
-        const float *wj = w + jj * mt;
-        const float4 *t = tmp + (size_t)i * cw + ts[jj];
-        float r = k[jj], g = r, b = r;
+        const int32_t n = T.n[jj], o0 = (int32_t)ky * IMG_SPAN + (n ? T.s[jj] - x0 : 0);
+        const float *wj = T.w + jj * IMG_MT_MAX;
+        float r = T.k[jj], g = r, b = r;
+#pragma unroll 8
         for (int32_t q = 0; q < n; q++) {
-            const float4 v = t[q];
             const float wq = wj[q];
-            r = __builtin_fmaf(wq, v.x, r);
-            g = __builtin_fmaf(wq, v.y, g);
-            b = __builtin_fmaf(wq, v.z, b);
+            r = __builtin_fmaf(wq, v[0][o0 + q], r);
+            g = __builtin_fmaf(wq, v[1][o0 + q], g);
+            b = __builtin_fmaf(wq, v[2][o0 + q], b);
         }
         uint16_t *o = band + (jj / 14) * IMG_PATCH + ky * 14 + jj % 14;
         o[0] = img_f16(__builtin_fminf(__builtin_fmaxf(b, -1.0f), 1.0f));
@@ -261,7 +317,7 @@ extern "C" int eva_img_over_white(void *rgba, size_t stride, uint32_t w, uint32_
 {
     if (!rgba || !w || !h || stride < (size_t)w * 4 || (stride & 3) || ((uintptr_t)rgba & 3))
         return xt_fail("eva_img_over_white", "bad image (4-byte aligned rows of w RGBA pixels)");
-    hipLaunchKernelGGL(k_img_over_white, dim3((w + 255) / 256, h), dim3(256), 0, (hipStream_t)stream, (uint8_t *)rgba,
+    hipLaunchKernelGGL(k_img_over_white, dim3((w + 255) / 256, (h + 3) / 4), dim3(256), 0, (hipStream_t)stream, (uint8_t *)rgba,
                        stride, w, h);
     return xt_check("eva_img_over_white");
 }
@@ -318,7 +374,7 @@ extern "C" int eva_img_pyramid(eva_pyr *p, void *levels, size_t bytes, uint32_t 
     return xt_check("eva_img_pyramid");
 }
 
-// scratch: tmp [S][cw] float4 of the vertical pass
+// scratch that the interface asks for: [S][cw] float4
 static size_t img_scratch(uint32_t S, uint32_t cw) { return (size_t)S * cw * 16; }
 
 extern "C" size_t eva_img_prep_bytes(uint32_t S, uint32_t max_side)
@@ -327,9 +383,10 @@ extern "C" size_t eva_img_prep_bytes(uint32_t S, uint32_t max_side)
     return img_scratch(S, max_side);
 }
 
-// pi_prep with the vertical pass staged in `scratch` (bytes long); what names the entry point in errors
+// pi_prep. The resample stages nothing in memory; `scratch` and its size are checked as the interface says. what names
+// the entry point in errors
 static int img_prep(const char *what, const eva_pyr *p, uint32_t x0, uint32_t y0, uint32_t cw, uint32_t ch, uint32_t S,
-                    void *scratch, size_t bytes, void *out, void *stream)
+                    const void *scratch, size_t bytes, void *out, void *stream)
 {
     if (!S) S = EVA_S;
     if (!p || !p->nlv || p->nlv > EVA_PYR_LV || !p->lv[0]) return xt_fail(what, "no pyramid");
@@ -363,9 +420,7 @@ static int img_prep(const char *what, const eva_pyr *p, uint32_t x0, uint32_t y0
     if (!scratch || bytes < img_scratch(S, cw) || ((uintptr_t)scratch & 15))
         return xt_fail(what, "scratch must be 16-byte aligned and hold S x (rect width on its level) x 16 bytes "
                              "(eva_img_prep_bytes(S, side); EVA_IMG_STATIC_BYTES for eva_img_prep_static)");
-    float4 *tmp = (float4 *)scratch;
-    hipLaunchKernelGGL(k_img_vpass, dim3((cw + 255) / 256, S), dim3(256), 0, st, src, stride, cw, ch, S, side, mt, tmp);
-    hipLaunchKernelGGL(k_img_hpass, bands, dim3(14 * 14 * IMG_BAND_P), 0, st, (const float4 *)tmp, cw, S, side, mt,
+    hipLaunchKernelGGL(k_img_resample, bands, dim3(IMG_RT), 0, st, src, stride, cw, ch, S, side, mt,
                        (uint16_t *)out);
     return xt_check(what);
 }
@@ -376,36 +431,10 @@ extern "C" int eva_img_prep(const eva_pyr *p, uint32_t x0, uint32_t y0, uint32_t
     return img_prep("eva_img_prep", p, x0, y0, cw, ch, S, scratch, bytes, out, stream);
 }
 
-// ---- eva_img_prep without a scratch argument, for callers that cannot allocate. The vertical pass is staged in
-// img_static, a file-scope device array (one copy per GPU, held until the process ends). In host code the array's name
-// is only a stand-in: its device address on the current GPU comes from hipGetSymbolAddress, taken once per device on
-// that device's first call and kept in img_static_dev. Every element the horizontal pass reads was written by the
-// vertical pass of the same call, so nothing needs clearing between calls; calls that overlap on one GPU race.
-static __device__ __align__(256) uint8_t img_static[EVA_IMG_STATIC_BYTES];
-#define IMG_MAX_DEVICES 64
-static void *img_static_dev[IMG_MAX_DEVICES];
-static pthread_mutex_t img_static_mu = PTHREAD_MUTEX_INITIALIZER;
-
-static void *img_static_addr(int dev)
-{
-    void *ptr;
-    pthread_mutex_lock(&img_static_mu);
-    ptr = img_static_dev[dev];
-    if (!ptr) {
-        if (hipGetSymbolAddress(&ptr, HIP_SYMBOL(img_static)) != hipSuccess) ptr = NULL;
-        img_static_dev[dev] = ptr;
-    }
-    pthread_mutex_unlock(&img_static_mu);
-    return ptr;
-}
-
+// ---- eva_img_prep without a scratch argument, up to the rects that EVA_IMG_STATIC_BYTES of scratch admitted when the
+// vertical pass was staged in memory
 extern "C" int eva_img_prep_static(const eva_pyr *p, uint32_t x0, uint32_t y0, uint32_t cw, uint32_t ch, uint32_t S,
                                    void *out, void *stream)
 {
-    int dev;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= IMG_MAX_DEVICES)
-        return xt_fail("eva_img_prep_static", "no current device");
-    void *ptr = img_static_addr(dev);
-    if (!ptr) return xt_fail("eva_img_prep_static", "hipGetSymbolAddress of the static scratch failed");
-    return img_prep("eva_img_prep_static", p, x0, y0, cw, ch, S, ptr, EVA_IMG_STATIC_BYTES, out, stream);
+    return img_prep("eva_img_prep_static", p, x0, y0, cw, ch, S, out, EVA_IMG_STATIC_BYTES, out, stream);
 }
