@@ -34,7 +34,7 @@ def _pieces(rows):
 
 
 @pytest.mark.parametrize("sparse", [False, True])
-@pytest.mark.parametrize("rows", [1, 65, 1408, 1409, 4096, 4097, 8192, 8200, 16400])
+@pytest.mark.parametrize("rows", [1, 65, 1408, 1409, 2817, 4096, 4097, 4353, 8192, 8200, 16400])
 def test_rows_do_not_depend_on_the_tile(dev, xt, rows, sparse):
     print(f"tile configurations: {rows} rows, sparse {sparse}", flush=True)
     L, P, st = xt.lib, xt.ptr, torch.cuda.current_stream().cuda_stream
