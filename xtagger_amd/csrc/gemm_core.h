@@ -30,9 +30,6 @@
 typedef __attribute__((address_space(3))) void lds_void;
 typedef int v4i __attribute__((ext_vector_type(4)));
 
-#ifndef XT_LAG
-#define XT_LAG 2      // MFMA -> promotion distance of the main-loop software pipeline
-#endif
 #ifndef XT_GM
 #define XT_GM 8       // grouped raster: row tiles walked together
 #endif
@@ -204,55 +201,13 @@ __device__ __forceinline__ void bs_wave_origin(int &wm0, int &wn0)
     wn0 = (w % C::NWN) * C::WN;
 }
 
-// One K step on a resident stage: TM x TN MFMAs, each block partial promoted into acc.
-template <class C>
-__device__ __forceinline__ void bs_step(const uint8_t *st, int wm0, int wn0, v4f (&acc)[C::TM][C::TN])
-{
-    const int lane = threadIdx.x & 63, g = lane >> 4;
-    const uint8_t *ta = st, *tb = st + C::A_BYTES;
-    const float *ts = (const float *)(st + C::A_BYTES + C::B_BYTES);
-    const float swv = *(const float *)(st + C::A_BYTES + C::B_BYTES + C::S_BYTES + 4 * (wn0 >> 7));
-    v8i a[C::TM];
-    v4f sc[C::TM];
-    v8i bcur = ld_frag(tb, wn0), bnext = bcur;
-#pragma unroll
-    for (int i = 0; i < C::TM; i++) a[i] = ld_frag(ta, wm0 + 16 * i);
-#pragma unroll
-    for (int i = 0; i < C::TM; i++) {
-        const float4 s4 = *(const float4 *)(ts + wm0 + 16 * i + 4 * g);
-        sc[i] = v4f{s4.x * swv, s4.y * swv, s4.z * swv, s4.w * swv};
-    }
-    // Software pipeline over the TN x TM MFMAs: MFMA number t is issued, then the four promotion fmas of MFMA
-    // t - LAG, whose result has had LAG MFMA slots to land; B fragments are read one column tile ahead.
-    constexpr int NS = C::TN * C::TM, LAG = XT_LAG;
-    v4f pr[LAG + 1];
-#pragma unroll
-    for (int t = 0; t < NS + LAG; t++) {
-        if (t < NS) {
-            const int j = t / C::TM, i = t % C::TM;
-            if (i == 0 && j + 1 < C::TN) bnext = ld_frag(tb, wn0 + 16 * (j + 1));
-            pr[t % (LAG + 1)] = mfma_e4m3_16x16x128(a[i], bcur);
-            if (i == C::TM - 1) bcur = bnext;
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // 1 MFMA
-        }
-        if (t >= LAG) {
-            const int u = t - LAG, j = u / C::TM, i = u % C::TM;
-            const v4f p = pr[u % (LAG + 1)];
-            acc[i][j][0] = __builtin_fmaf(p[0], sc[i][0], acc[i][j][0]);
-            acc[i][j][1] = __builtin_fmaf(p[1], sc[i][1], acc[i][j][1]);
-            acc[i][j][2] = __builtin_fmaf(p[2], sc[i][2], acc[i][j][2]);
-            acc[i][j][3] = __builtin_fmaf(p[3], sc[i][3], acc[i][j][3]);
-            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);  // then 4 VALU
-        }
-    }
-}
-
 // Wave tiles that the fixed-order step serves
 template <class C>
 constexpr bool BsFixed = (C::TM == 4 || C::TM == 2) && (C::TN == 8 || C::TN == 4 || C::TN == 2);
 
-// The same K step for 64 x 128 and 64 x 64 wave tiles (TM = 4, TN = 8 or 4) in a fixed issue order (for 64 x 64, the
-// single GEMM's 128 x 128 tiles, 12% faster than bs_step at M = 1025). The matrix-core instructions and
+// One K step on a resident stage, TM x TN MFMAs with each block partial promoted into acc, for wave tiles of 4 or 2 row
+// tiles in a fixed issue order (for 64 x 64 wave tiles 12% faster at M = 1025 than the order the compiler gives it). The schedule is written for 64 x 128; a smaller tile puts several of the stage's loads after
+// one MFMA (PER) where it has fewer MFMAs than loads. The matrix-core instructions and
 // the promotion fmas are single-instruction asm statements, and every LDS read sits between them, so the compiler
 // keeps the written order (it still allocates registers and places the LDS waits):
 //  - A 0 and B 0 are read first, then the scales, then A 1-3 and B 1: the first MFMA waits for four reads only;
@@ -477,36 +432,29 @@ __device__ __forceinline__ void bs_mainloop(const uint8_t *__restrict__ A, int l
             is = is == C::NS - 1 ? 0 : is + 1;
         }
     };
-    if constexpr (BsFixed<C>) {
-        if (live > 8 * C::TM) {
-            v4f pr[4];          // the MFMA result ring, and the scales of the last step's last three MFMAs (their
-            float scp[3][4];    // promotions run at the start of the next step)
-            int kbi = 0;
-            kloop([&](const uint8_t *st, uint32_t dst, int dkb) {
-                bs_step_fixed<C, TR>(st, wm0, wn0, acc, op, dst, dkb, pr, scp, kbi > 0);
-                kbi++;
-            });
-            asm volatile("s_nop 7\n\ts_nop 7" ::: "memory");  // 12+ wait states after the last MFMA
-            bs_step_fixed_flush<C, TR>(acc, pr, scp);
-        } else if (C::TM == 4 && live > 16)
-            kloop([&](const uint8_t *st, uint32_t dst, int dkb) {
-                bs_step_rows<C, C::TM / 2, TR>(st, wm0, wn0, acc, op, dst, dkb);
-            });
-        else if (live > 0)
-            kloop([&](const uint8_t *st, uint32_t dst, int dkb) {
-                bs_step_rows<C, 1, TR>(st, wm0, wn0, acc, op, dst, dkb);
-            });
-        else
-            kloop([&](const uint8_t *, uint32_t dst, int dkb) {
-                if (dkb >= 0) op.issue(dst, dkb);
-            });
-    } else {
-        static_assert(!TR, "the transposed tile needs the fixed-order steps");
+    static_assert(BsFixed<C>, "wave tiles of 4 or 2 row tiles");
+    if (live > 8 * C::TM) {
+        v4f pr[4];          // the MFMA result ring, and the scales of the last step's last three MFMAs (their
+        float scp[3][4];    // promotions run at the start of the next step)
+        int kbi = 0;
         kloop([&](const uint8_t *st, uint32_t dst, int dkb) {
-            if (dkb >= 0) op.issue(dst, dkb);
-            bs_step<C>(st, wm0, wn0, acc);
+            bs_step_fixed<C, TR>(st, wm0, wn0, acc, op, dst, dkb, pr, scp, kbi > 0);
+            kbi++;
         });
-    }
+        asm volatile("s_nop 7\n\ts_nop 7" ::: "memory");  // 12+ wait states after the last MFMA
+        bs_step_fixed_flush<C, TR>(acc, pr, scp);
+    } else if (C::TM == 4 && live > 16)
+        kloop([&](const uint8_t *st, uint32_t dst, int dkb) {
+            bs_step_rows<C, C::TM / 2, TR>(st, wm0, wn0, acc, op, dst, dkb);
+        });
+    else if (live > 0)
+        kloop([&](const uint8_t *st, uint32_t dst, int dkb) {
+            bs_step_rows<C, 1, TR>(st, wm0, wn0, acc, op, dst, dkb);
+        });
+    else
+        kloop([&](const uint8_t *, uint32_t dst, int dkb) {
+            if (dkb >= 0) op.issue(dst, dkb);
+        });
     lds_barrier();
 }
 
