@@ -218,3 +218,26 @@ def test_no_scratch(tmp_path, src):
     bad = {k: v for k, v in res.items() if v[1] or v[2]}
     assert not bad, f"kernels with spills or scratch in {src}: {bad}"
 
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
+def test_qkv_v_stores_step_by_constants(tmp_path):
+    """Each lane of k_qkv writes its token's dims of v^T one 2-byte store at a time, a constant number of bytes apart:
+    their addresses come from additions. A full 64-bit multiply per store (a loop that starts at a per-lane dim) shows as
+    at least as many v_mad_u64_u32 as stores; the tile's own addressing needs far fewer."""
+    asm = tmp_path / "layer.s"
+    cmd = [HIPCC] + FLAGS + ["-I" + os.path.join(os.path.dirname(CSRC), "..", "include"), "-I" + CSRC,
+                             os.path.join(CSRC, "layer.hip"), "-o", str(asm)]
+    r = subprocess.run(cmd, capture_output=True, text=True, timeout=600)
+    assert r.returncode == 0, r.stderr[-2000:]
+    seen, cur = {}, None
+    for line in asm.read_text().splitlines():
+        m = re.match(r"(_Z\w+):", line)
+        if m:
+            cur = m.group(1) if "k_qkv" in m.group(1) else None
+        elif cur and line.strip().startswith(("v_mad_u64_u32", "global_store_short")):
+            c = seen.setdefault(cur, [0, 0])
+            c[line.strip().startswith("global_store_short")] += 1
+    assert len(seen) == 4, sorted(seen)                       # two tiles, dense and 2:4-sparse
+    bad = {k: v for k, v in seen.items() if v[0] >= v[1]}
+    assert not bad, f"(v_mad_u64_u32, v stores) per kernel: {bad}"

@@ -33,9 +33,10 @@ __global__ void __launch_bounds__(C::NT) k_qkv(const uint8_t *__restrict__ h8, c
     const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
     const int part = n0 >> 10, head0 = ((n0 & 1023) + wn0) >> 6;
     // v: the wave's rows x dims (one or two heads) are transposed through its own LDS slice ([WN dims][WM + 4] bf16,
-    // padded rows), then lanes walk rows (consecutive tokens; two dims at a time where the wave has 32 rows). The slice takes the tile in whichever layout the main
-    // loop leaves it: the sparse loop's transposed tile directly (no pass through the dense layout first), the dense
-    // tile as one 8-byte write of four consecutive tokens per (row tile, column tile).
+    // padded rows), then lanes walk rows (consecutive tokens; two dims at a time where the wave has 32 rows, the lane's
+    // own dim folded into its base pointers so that the loop steps both by constants). The slice takes the tile in
+    // whichever layout the main loop leaves it: the sparse loop's transposed tile directly (no pass through the dense
+    // layout first), the dense tile as one 8-byte write of four consecutive tokens per (row tile, column tile).
     uint16_t *tr = (uint16_t *)(smem + (threadIdx.x >> 6) * LayerMem<C>::TRSLICE);
     auto v_out = [&]() {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -43,11 +44,12 @@ __global__ void __launch_bounds__(C::NT) k_qkv(const uint8_t *__restrict__ h8, c
         const int row = lane % C::WM, d0 = lane / C::WM, m = m0 + wm0 + row;
         if (m < rows) {
             const int b = m / XT_T, t = m - b * XT_T;
+            const uint16_t *src = tr + d0 * TRLD + row;
 #pragma unroll
             for (int hh = 0; hh < NH; hh++) {
-                uint16_t *dst = vt + ((size_t)b * XT_NH + head0 + hh) * XT_HD * XT_TP + t;
+                uint16_t *dst = vt + (((size_t)b * XT_NH + head0 + hh) * XT_HD + d0) * XT_TP + t;
 #pragma unroll 8
-                for (int d = d0; d < XT_HD; d += DS) dst[(size_t)d * XT_TP] = tr[(64 * hh + d) * TRLD + row];
+                for (int d = 0; d < XT_HD; d += DS) dst[(size_t)d * XT_TP] = src[(64 * hh + d) * TRLD];
             }
         }
     };
