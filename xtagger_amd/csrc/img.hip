@@ -383,10 +383,16 @@ extern "C" size_t eva_img_prep_bytes(uint32_t S, uint32_t max_side)
     return img_scratch(S, max_side);
 }
 
-// pi_prep. The resample stages nothing in memory; `scratch` and its size are checked as the interface says. what names
-// the entry point in errors
-static int img_prep(const char *what, const eva_pyr *p, uint32_t x0, uint32_t y0, uint32_t cw, uint32_t ch, uint32_t S,
-                    const void *scratch, size_t bytes, void *out, void *stream)
+// A crop on its level: the host part of pi_prep (pi_level, pi_lsrc) and the limits that both entry points share. what
+// names the entry point in errors; an S of 0 becomes the default side.
+struct ImgRect {
+    const uint8_t *src;
+    size_t stride;
+    uint32_t cw, ch, side, S;
+};
+
+static int img_rect(const char *what, const eva_pyr *p, uint32_t x0, uint32_t y0, uint32_t cw, uint32_t ch, uint32_t S,
+                    const void *out, ImgRect &r)
 {
     if (!S) S = EVA_S;
     if (!p || !p->nlv || p->nlv > EVA_PYR_LV || !p->lv[0]) return xt_fail(what, "no pyramid");
@@ -404,37 +410,51 @@ static int img_prep(const char *what, const eva_pyr *p, uint32_t x0, uint32_t y0
     y0 >>= L;
     x0 = x0 < p->lw[L] ? x0 : p->lw[L] - 1;
     y0 = y0 < p->lh[L] ? y0 : p->lh[L] - 1;
-    cw = x1 > x0 ? x1 - x0 : 1;
-    ch = y1 > y0 ? y1 - y0 : 1;
-    const uint8_t *src = p->lv[L] + (size_t)y0 * p->ls[L] + (size_t)x0 * 4;
-    const size_t stride = p->ls[L];
-    const uint32_t side = cw > ch ? cw : ch, pr = S / 14;
+    r.cw = x1 > x0 ? x1 - x0 : 1;
+    r.ch = y1 > y0 ? y1 - y0 : 1;
+    r.src = p->lv[L] + (size_t)y0 * p->ls[L] + (size_t)x0 * 4;
+    r.stride = p->ls[L];
+    r.side = r.cw > r.ch ? r.cw : r.ch;
+    r.S = S;
+    if (r.side != S && img_mt(r.side, S) > IMG_MT_MAX)
+        return xt_fail(what, "rect more than 5x the model side on its level");
+    return 0;
+}
+
+// pi_prep of a checked rect: the identity where its long side is S, else the resample (which stages nothing in memory)
+static int img_prep(const char *what, const ImgRect &r, void *out, void *stream)
+{
+    const uint32_t pr = r.S / 14;
     const dim3 bands((pr + IMG_BAND_P - 1) / IMG_BAND_P, pr);
-    hipStream_t st = (hipStream_t)stream;
-    if (side == S) {
-        hipLaunchKernelGGL(k_img_ident, bands, dim3(256), 0, st, src, stride, cw, ch, S, (uint16_t *)out);
-        return xt_check(what);
-    }
-    const uint32_t mt = img_mt(side, S);
-    if (mt > IMG_MT_MAX) return xt_fail(what, "rect more than 5x the model side on its level");
-    if (!scratch || bytes < img_scratch(S, cw) || ((uintptr_t)scratch & 15))
-        return xt_fail(what, "scratch must be 16-byte aligned and hold S x (rect width on its level) x 16 bytes "
-                             "(eva_img_prep_bytes(S, side); EVA_IMG_STATIC_BYTES for eva_img_prep_static)");
-    hipLaunchKernelGGL(k_img_resample, bands, dim3(IMG_RT), 0, st, src, stride, cw, ch, S, side, mt,
-                       (uint16_t *)out);
+    if (r.side == r.S)
+        hipLaunchKernelGGL(k_img_ident, bands, dim3(256), 0, (hipStream_t)stream, r.src, r.stride, r.cw, r.ch, r.S,
+                           (uint16_t *)out);
+    else
+        hipLaunchKernelGGL(k_img_resample, bands, dim3(IMG_RT), 0, (hipStream_t)stream, r.src, r.stride, r.cw, r.ch, r.S,
+                           r.side, img_mt(r.side, r.S), (uint16_t *)out);
     return xt_check(what);
 }
 
+// The scratch of a resampled rect is checked as the interface says and passed no further.
 extern "C" int eva_img_prep(const eva_pyr *p, uint32_t x0, uint32_t y0, uint32_t cw, uint32_t ch, uint32_t S,
                             void *scratch, size_t bytes, void *out, void *stream)
 {
-    return img_prep("eva_img_prep", p, x0, y0, cw, ch, S, scratch, bytes, out, stream);
+    ImgRect r;
+    if (img_rect("eva_img_prep", p, x0, y0, cw, ch, S, out, r)) return -1;
+    if (r.side != r.S && (!scratch || bytes < img_scratch(r.S, r.cw) || ((uintptr_t)scratch & 15)))
+        return xt_fail("eva_img_prep", "scratch must be 16-byte aligned and hold S x (rect width on its level) x 16 "
+                                       "bytes (eva_img_prep_bytes(S, side))");
+    return img_prep("eva_img_prep", r, out, stream);
 }
 
-// ---- eva_img_prep without a scratch argument, up to the rects that EVA_IMG_STATIC_BYTES of scratch admitted when the
-// vertical pass was staged in memory
+// ---- eva_img_prep without a scratch argument, for rects whose scratch would fit EVA_IMG_STATIC_BYTES
 extern "C" int eva_img_prep_static(const eva_pyr *p, uint32_t x0, uint32_t y0, uint32_t cw, uint32_t ch, uint32_t S,
                                    void *out, void *stream)
 {
-    return img_prep("eva_img_prep_static", p, x0, y0, cw, ch, S, out, EVA_IMG_STATIC_BYTES, out, stream);
+    ImgRect r;
+    if (img_rect("eva_img_prep_static", p, x0, y0, cw, ch, S, out, r)) return -1;
+    if (r.side != r.S && img_scratch(r.S, r.cw) > EVA_IMG_STATIC_BYTES)
+        return xt_fail("eva_img_prep_static", "rect too wide: S x (its width on its level) x 16 is more than "
+                                              "EVA_IMG_STATIC_BYTES");
+    return img_prep("eva_img_prep_static", r, out, stream);
 }
