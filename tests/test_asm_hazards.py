@@ -208,7 +208,7 @@ def _resources(tmp_path, src):
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
-@pytest.mark.parametrize("src", ["layer.hip", "px.hip", "quant.hip", "attn.hip", "norm.hip"])
+@pytest.mark.parametrize("src", ["layer.hip", "px.hip", "quant.hip", "attn.hip", "norm.hip", "img.hip"])
 def test_no_scratch(tmp_path, src):
     """No kernel spills registers or keeps an array in scratch memory: a dynamically indexed accumulator array, or
     two main loops whose registers the allocator cannot keep apart, silently moves the accumulators to memory and

@@ -539,7 +539,7 @@ def test_patch_embed(dev, xt, orc):
 def test_partial_row_tile_bit_identical(dev, xt, orc, tail):
     """A last row tile with `tail` rows below M (its waves run only the 16-row tiles that hold such rows) gives its
     rows bit for bit what a whole tile gives them: oproj and fc1 over M = 2048 + tail rows against the same rows of an
-    M = 2304 run (nine whole tiles)."""
+    M = 2304 run (whole tiles of every height). The tiles of other row counts: test_tile_configs_gpu.py."""
     MF, MT = 2304, 2048 + tail
     _say(f"partial row tile of {tail} rows")
     _, qa, sa = _packed_act(orc, MF, D, 71)
@@ -578,7 +578,7 @@ def test_partial_row_tile_bit_identical(dev, xt, orc, tail):
 @pytest.mark.parametrize("tail", [8, 32])
 def test_partial_row_tile_bit_identical_fc2(dev, xt, orc, tail):
     """fc2 (its row statistics and column terms staged while the first operands load) over M = 2048 + tail rows
-    against the same rows of a nine-tile run."""
+    against the same rows of an M = 2304 run (whole tiles)."""
     MF, MT = 2304, 2048 + tail
     r = np.random.default_rng(81)
     h = (r.standard_normal((MF, HIDP)) * 0.3).astype(np.float32)

@@ -1,7 +1,8 @@
 """The layer GEMMs choose their tile by the number of rows. Every output takes its K blocks in the same order whatever
 the tile, so a row's result must not depend on it: each kernel over `rows` rows, on both sides of every limit of the
-rules, against the same rows taken in pieces of at most 1025 (which run the smallest tiles, and which the parity tests
-check against the oracle), bit for bit."""
+rules (test_tile_rules.py checks on the host that the row counts here are), against the same rows taken in pieces of at
+most 1025 (which run the smallest tiles, and which the parity tests check against the oracle), bit for bit. The pieces
+go past `rows` and start elsewhere than the call's tiles, so every row sits in another place of another launch."""
 import pytest
 import torch
 
@@ -29,29 +30,52 @@ class _W:
         return (X.ptr(self.v),) + ((X.ptr(self.x),) if self.x is not None else ()) + (X.ptr(self.s),)
 
 
+PAST = 129   # rows that the operands hold past `rows`
+
+
 def _pieces(rows):
-    return [(r, min(r + T, rows)) for r in range(0, rows, T)]
+    """[0, 700) and then steps of 1025, to PAST rows past `rows`"""
+    edges = [0, *range(700, rows + PAST, T), rows + PAST]
+    return list(zip(edges[:-1], edges[1:]))
+
+
+RES_ROWS = [1, 65, 1408, 1409, 2817, 4096, 4097, 4353, 8192, 8193, 8200, 8447, 8448, 10250, 16384, 16400]
+TAIL_BASES, TAILS = [1280, 2048, 4224, 10240], [1, 8, 16, 17, 32, 33, 48, 49, 64]
 
 
 @pytest.mark.parametrize("sparse", [False, True])
-@pytest.mark.parametrize("rows", [1, 65, 1408, 1409, 2817, 4096, 4097, 4353, 8192, 8200, 16400])
+@pytest.mark.parametrize("rows", RES_ROWS)
 def test_rows_do_not_depend_on_the_tile(dev, xt, rows, sparse):
+    _check_rows(dev, xt, rows, sparse)
+
+
+@pytest.mark.parametrize("sparse", [False, True])
+@pytest.mark.parametrize("base", TAIL_BASES)
+def test_partial_row_tiles_of_every_tile(dev, xt, base, sparse):
+    """a last row tile with 1 to 64 rows below M (a wave runs only the 16-row tiles that hold such rows), at row counts
+    that take fc1's smaller tile and each of the three tiles of the out-projection and fc2"""
+    for tail in TAILS:
+        _check_rows(dev, xt, base + tail, sparse)
+
+
+def _check_rows(dev, xt, rows, sparse):
     print(f"tile configurations: {rows} rows, sparse {sparse}", flush=True)
     L, P, st = xt.lib, xt.ptr, torch.cuda.current_stream().cuda_stream
     sfx = "_sp" if sparse else ""
     g = torch.Generator(device=dev)
     g.manual_seed(rows)
-    lds = rows + 256             # a piece's last tile reads scales (of rows it drops) up to 127 rows past its own
-    h8, hs = _codes(g, dev, rows, D), torch.rand(8, lds, generator=g, device=dev) * 0.01
-    m8, ms = _codes(g, dev, rows, HIDP), torch.rand(22, lds, generator=g, device=dev) * 0.01
+    R = rows + PAST
+    lds = R + 256                # a piece's last tile reads scales (of rows it drops) up to 127 rows past its own
+    h8, hs = _codes(g, dev, R, D), torch.rand(8, lds, generator=g, device=dev) * 0.01
+    m8, ms = _codes(g, dev, R, HIDP), torch.rand(22, lds, generator=g, device=dev) * 0.01
     stat = torch.rand(22, lds, 2, generator=g, device=dev) * 20
-    x0 = torch.randn(rows, D, generator=g, device=dev).half()
+    x0 = torch.randn(R, D, generator=g, device=dev).half()
     cn, dn = torch.rand(D, generator=g, device=dev), torch.rand(D, generator=g, device=dev)
     wo, w1, w2 = (_W(g, dev, *s, sparse) for s in ((D, D), (2 * HIDP, D), (D, HIDP)))
 
     def run(bounds):
         xo, xf = x0.clone(), x0.clone()
-        mo, so, to = (torch.zeros(rows, HIDP, dtype=U8, device=dev), torch.zeros(22, lds, device=dev),
+        mo, so, to = (torch.zeros(R, HIDP, dtype=U8, device=dev), torch.zeros(22, lds, device=dev),
                       torch.zeros(22, lds, 2, device=dev))
         for a, b in bounds:
             n = b - a
@@ -63,12 +87,15 @@ def test_rows_do_not_depend_on_the_tile(dev, xt, rows, sparse):
         torch.cuda.synchronize()
         return xo, xf, mo, so, to
 
-    for got, ref in zip(run([(0, rows)]), run(_pieces(rows))):
-        assert torch.equal(got, ref)
+    (xo, xf, mo, so, to), (rxo, rxf, rmo, rso, rto) = run([(0, rows)]), run(_pieces(rows))
+    for got, ref, first in ((xo, rxo, x0), (xf, rxf, x0), (mo, rmo, torch.zeros_like(mo))):
+        assert torch.equal(got[:rows], ref[:rows]) and torch.equal(got[rows:], first[rows:])   # nothing past the rows
+    for got, ref in ((so, rso), (to, rto)):
+        assert torch.equal(got[:, :rows], ref[:, :rows]) and not got[:, rows:].any()
 
 
 @pytest.mark.parametrize("sparse", [False, True])
-@pytest.mark.parametrize("nb", [2, 3, 6, 7])
+@pytest.mark.parametrize("nb", [2, 3, 5, 6, 7])
 def test_qkv_rows_do_not_depend_on_the_tile(dev, xt, nb, sparse):
     print(f"qkv tile configurations: {nb} images, sparse {sparse}", flush=True)
     L, P, st = xt.lib, xt.ptr, torch.cuda.current_stream().cuda_stream
@@ -216,3 +243,32 @@ def test_px_fc1_rows_do_not_depend_on_the_tile(dev, xt, rows, with_rs):
 
     for got, ref in zip(run(rows), run(1000)):
         assert torch.equal(got, ref)
+
+
+PX_ROWS = [1, 65, 4096, 4097, 8192, 8193, 8447, 8448, 10273, 16384]
+
+
+@pytest.mark.parametrize("rows", PX_ROWS)
+def test_px_residual_rows_do_not_depend_on_the_tile(dev, xt, rows):
+    """PixAI's out-projection (K = 1024) and fc2 (K = 4736) on both sides of the limits of their tiles"""
+    print(f"px residual GEMMs: {rows} rows", flush=True)
+    L, P, st = xt.lib, xt.ptr, torch.cuda.current_stream().cuda_stream
+    g = torch.Generator(device=dev)
+    g.manual_seed(rows)
+    R = rows + PAST
+    lds = R + 256
+    for fn, K in ((L.px_k_proj, D), (L.px_k_fc2, PXH)):
+        a8, as_ = _codes(g, dev, R, K), torch.rand(K // 128, lds, generator=g, device=dev) * 0.01
+        w, bias = _W(g, dev, D, K, False), torch.randn(D, generator=g, device=dev)
+        x0 = torch.randn(R, D, generator=g, device=dev).half()
+
+        def run(bounds):
+            x = x0.clone()
+            for a, b in bounds:
+                assert fn(P(a8[a:]), P(as_.reshape(-1)[a:]), lds, *w.args(xt), P(bias), P(x[a:]), b - a, st) == 0
+            torch.cuda.synchronize()
+            return x
+
+        got, ref = run([(0, rows)]), run(_pieces(rows))
+        assert torch.equal(got[:rows], ref[:rows]) and torch.equal(got[rows:], x0[rows:])
+        assert not torch.equal(got[:rows], x0[:rows])

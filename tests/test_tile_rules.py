@@ -1,0 +1,87 @@
+"""Which tile each launcher's rule picks, asked of the rules themselves (the kernel sources compiled into small libraries
+with one query function each), so that the row counts of test_tile_configs_gpu.py cannot drift away from the limits they
+are there for. CPU only."""
+import concurrent.futures
+import ctypes as C
+import os
+import shutil
+import subprocess
+
+import pytest
+
+from tests import test_tile_configs_gpu as G
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "xtagger_amd", "csrc")
+HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+pytestmark = pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
+
+# (source, the expression that calls its rule with a generic lambda f)
+RULES = {"res": ("layer.hip", "with_res_cfg(a, b, f)"), "qkv": ("layer.hip", "with_qkv_cfg(a, f)"),
+         "fc1": ("layer.hip", "with_fc1_cfg(a, f)"), "pe": ("layer.hip", "with_pe_cfg(a, f)"),
+         "px_fc1": ("px.hip", "with_px_fc1_cfg(a, f)"), "gemm": ("quant.hip", "with_gemm_cfg(a, b, f)")}
+
+
+@pytest.fixture(scope="module")
+def tile(tmp_path_factory):
+    """tile(rule, a, b=0) -> (BM, BN)"""
+    d = tmp_path_factory.mktemp("rules")
+
+    def build(src):
+        body = "".join(f'extern "C" int rule_{k}(int a, int b) {{ int t = 0; auto f = [&](auto c) {{ using T = '
+                       f'decltype(c); t = 1000 * T::BM + T::BN; }}; {e}; return t; }}\n'
+                       for k, (s, e) in RULES.items() if s == src)
+        f = d / ("q_" + src)
+        f.write_text(f'#include "{os.path.join(CSRC, src)}"\n{body}')
+        so = str(f) + ".so"
+        r = subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared", "-ffp-contract=off",
+                            "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-I" + CSRC,
+                            "-I" + os.path.join(CSRC, "..", "..", "include"), str(f), "-o", so],
+                           capture_output=True, text=True, timeout=600)
+        assert r.returncode == 0, r.stderr[-2000:]
+        return src, C.CDLL(so)
+
+    with concurrent.futures.ThreadPoolExecutor(3) as ex:
+        libs = dict(ex.map(build, sorted({s for s, _ in RULES.values()})))
+    return lambda rule, a, b=0: divmod(getattr(libs[RULES[rule][0]], "rule_" + rule)(a, b), 1000)
+
+
+def _limits(tile, rule, hi, *args):
+    """the rows r in 1 .. hi - 1 after which the tile changes"""
+    t = [tile(rule, r, *args) for r in range(1, hi + 1)]
+    return [r for r in range(1, hi) if t[r - 1] != t[r]]
+
+
+SML, MID, BIG = (64, 128), (128, 128), (256, 256)
+
+
+def test_both_sides_of_every_limit(tile):
+    """every limit below the tested range's end has a tested row count on either side, without another limit between"""
+    def check(limits, rows, end):
+        edges = [0, *[x for x in limits if x < end], end]
+        for lo, hi in zip(edges[:-1], edges[1:]):
+            assert any(lo < r <= hi for r in rows), f"no tested row count in ({lo}, {hi}]"
+
+    assert _limits(tile, "res", 20000, G.HIDP) == _limits(tile, "res", 20000, G.PXH) == [4096, 8192]
+    k1024 = _limits(tile, "res", 20000, G.D)
+    assert k1024[:3] == [4096, 8447, 16384]
+    for limits, rows in ((k1024, G.RES_ROWS), ([4096, 8192], G.RES_ROWS), (k1024[:2], G.PX_ROWS), ([4096, 8192], G.PX_ROWS)):
+        check(limits, rows, 16400)
+        for x in limits[:2]:
+            assert x in rows and x + 1 in rows, x
+    assert _limits(tile, "fc1", 20000) == [1408] and {1408, 1409} <= set(G.RES_ROWS)
+    assert _limits(tile, "px_fc1", 20000) == [12288]
+    assert [tile("qkv", 1025 * nb) for nb in (1, 2, 3, 5, 6, 7, 8, 16, 32)] == [MID, MID, BIG, BIG, MID, BIG, BIG, BIG, BIG]
+    assert [tile("pe", r) for r in (1024, 2048, 2049, 3072)] == [(64, 64), (64, 64), MID, MID]
+
+
+def test_partial_row_tiles_cover_every_tile(tile):
+    for k in (G.D, G.HIDP):
+        assert [{tile("res", b + t, k) for t in G.TAILS} for b in G.TAIL_BASES[1:]] == [{SML}, {MID}, {BIG}], k
+    assert [{tile("fc1", b + t) for t in G.TAILS} for b in G.TAIL_BASES] == [{(128, 256)}, {BIG}, {BIG}, {BIG}]
+
+
+def test_gemm_shapes_cover_every_tile(tile):
+    shapes = next(m for m in G.test_gemm_any_alignment_and_tile.pytestmark if "M,N" in m.args[0]).args[1]
+    for sparse in (False, True):
+        got = {tile("gemm", M, (N + 15) // 16 * 16 if sparse else N) for M, N, *_ in shapes}
+        assert got == {(64, 64), SML, MID, BIG}, got
