@@ -234,8 +234,8 @@ size_t eva_img_pyramid_bytes(uint32_t w, uint32_t h, uint32_t S);
 /* pi_pyramid: levels 1.. of p into `levels` (32-byte aligned, eva_img_pyramid_bytes), 2x2 boxes of pi_half
  * (procimg.h:636-661); sets p->nlv and the level fields. */
 int eva_img_pyramid(eva_pyr *p, void *levels, size_t bytes, uint32_t S, void *stream);
-/* Scratch bytes that eva_img_prep asks for with crops whose long side on the chosen level is at most max_side (4 S - 1 covers
- * every crop of a full pyramid). */
+/* Scratch bytes that eva_img_prep asks for with crops whose long side on the chosen level is at most max_side (4 S - 1
+ * covers every crop of a full pyramid). */
 size_t eva_img_prep_bytes(uint32_t S, uint32_t max_side);
 /* pi_prep (procimg.h:926-969): the level-0 rect (x0, y0, cw, ch) -> out fp16 [(S/14)^2][592] (EVA_IN halves at
  * S = 448; 16-byte aligned), resampled (bicubic onto the white square, [-1, 1], BGR planes) from the level pi_level
@@ -245,8 +245,8 @@ int eva_img_prep(const eva_pyr *p, uint32_t x0, uint32_t y0, uint32_t cw, uint32
                  size_t bytes, void *out, void *stream);
 /* eva_img_prep that allocates nothing and takes no scratch argument. No counterpart in the reference: it is for callers
  * that cannot allocate (code under HIP graph capture, tight serving loops). Nothing is staged in memory, so calls on
- * several streams may overlap; rects whose chosen level would need more scratch than EVA_IMG_STATIC_BYTES (S x rect
- * width on the level x 16 bytes, i.e. the long side on the level below 4 S - 1 at S = 448) fail with -1. */
+ * several streams may overlap; rects that eva_img_prep would ask more scratch for than EVA_IMG_STATIC_BYTES (S x rect
+ * width on the level x 16 bytes: more than 4 S - 1 pixels wide there at S = 448) fail with -1. */
 #define EVA_IMG_STATIC_BYTES ((size_t)448 * (4 * 448 - 1) * 16)
 int eva_img_prep_static(const eva_pyr *p, uint32_t x0, uint32_t y0, uint32_t cw, uint32_t ch, uint32_t S, void *out,
                         void *stream);

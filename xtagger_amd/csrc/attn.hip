@@ -332,9 +332,11 @@ __global__ void __launch_bounds__(128 * QT) k_flash(const uint16_t *__restrict__
 }
 
 // Queries per block: 128 (QT = 4 query tiles of 32 per head, two waves per SIMD), or 64 while those blocks get a CU
-// each: a wave alone on its SIMD runs a key tile in 1.2 us, one of two in 1.4. us, 128 -> 64 queries: 23.8 -> 20.4 for
-// one sequence of 1025 (72 -> 136 blocks), 9.9 -> 8.3 for one of 200; with more blocks than CUs the halved reuse of
-// the K and V^T stages loses (two sequences of 1025: 24.8 -> 28.1; 18 of 576: 38.3 -> 48.0).
+// each: a wave alone on its SIMD runs a key tile in 1.2 us, one of two in 1.4. us a call, 128 -> 64 queries: 23.8 -> 20.4
+// for one sequence of 1025 (72 -> 136 blocks), 9.9 -> 8.3 for one of 200; with more blocks than CUs the halved reuse of
+// the K and V^T stages loses (two sequences of 1025: 24.8 -> 28.1; 18 of 576: 38.3 -> 48.0). All with k_flash<2> as its
+// launch bounds let it compile: a budget of more than 256 registers, which the compiler uses to keep the accumulators
+// in AGPRs and copies them for every key tile (240 of its 542 instructions; k_flash<4> takes 337 and none).
 template <int N>
 struct FaQt {
     static constexpr int value = N;

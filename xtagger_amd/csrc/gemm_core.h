@@ -67,9 +67,6 @@ struct BsCfg {
     static constexpr int LPS_SP = LA + 2 * LV + 1;
 };
 
-// 16-byte chunk swizzle of the attention and patch-embedding tiles (chunk c of row r at c ^ (r & 7))
-__device__ __forceinline__ uint32_t swz(int row, int chunk) { return (uint32_t)(row * 128 + ((chunk ^ (row & 7)) << 4)); }
-
 // Raw buffer descriptor (base, stride 0, num_records = bytes, 32-bit dword format) in SGPRs.
 __device__ __forceinline__ v4i buf_desc(const void *p, uint32_t bytes)
 {
@@ -206,10 +203,11 @@ template <class C>
 constexpr bool BsFixed = (C::TM == 4 || C::TM == 2) && (C::TN == 8 || C::TN == 4 || C::TN == 2);
 
 // One K step on a resident stage, TM x TN MFMAs with each block partial promoted into acc, for wave tiles of 4 or 2 row
-// tiles in a fixed issue order (for 64 x 64 wave tiles 12% faster at M = 1025 than the order the compiler gives it). The schedule is written for 64 x 128; a smaller tile puts several of the stage's loads after
-// one MFMA (PER) where it has fewer MFMAs than loads. The matrix-core instructions and
-// the promotion fmas are single-instruction asm statements, and every LDS read sits between them, so the compiler
-// keeps the written order (it still allocates registers and places the LDS waits):
+// tiles in a fixed issue order (for 64 x 64 wave tiles 12% faster at M = 1025 than the order the compiler gives it). The
+// schedule is written for 64 x 128; a smaller tile puts several of the stage's loads after one MFMA (PER) where it has
+// fewer MFMAs than loads. The matrix-core instructions and the promotion fmas are single-instruction asm statements, and
+// every LDS read sits between them, so the compiler keeps the written order (it still allocates registers and places the
+// LDS waits):
 //  - A 0 and B 0 are read first, then the scales, then A 1-3 and B 1: the first MFMA waits for four reads only;
 //  - B fragment j + 2 is read right after MFMA (j, 0), into the slot B fragment j - 1 has left (3-slot ring);
 //  - the promotion of MFMA t - 3 follows MFMA t (15 instructions separate an MFMA from the first VALU read of its
@@ -384,10 +382,10 @@ struct BsNoPre {
     __device__ __forceinline__ void operator()() const {}
 };
 
-// Main loop (SKIP: waves whose rows are all past M skip their matrix work). On return acc[i][j][r] holds output row m0 + wm0 + 16 i + 4 (lane >> 4) + r, column
-// n0 + wn0 + 16 j + (lane & 15), where (wm0, wn0) = bs_wave_origin(); with TR the tile transposed (the MFMAs take
-// the weights as A): row m0 + wm0 + 16 i + (lane & 15), column n0 + wn0 + 16 j + 4 (lane >> 4) + r, one row scale
-// per lane and row tile. The block is synchronised, no load is in
+// Main loop (SKIP: waves whose rows are all past M skip their matrix work). On return acc[i][j][r] holds output row
+// m0 + wm0 + 16 i + 4 (lane >> 4) + r, column n0 + wn0 + 16 j + (lane & 15), where (wm0, wn0) = bs_wave_origin(); with
+// TR the tile transposed (the MFMAs take the weights as A): row m0 + wm0 + 16 i + (lane & 15), column
+// n0 + wn0 + 16 j + 4 (lane >> 4) + r, one row scale per lane and row tile. The block is synchronised, no load is in
 // flight and the whole shared memory is free for the epilogue. pre() runs once the first stages' loads are issued
 // (epilogue inputs can be fetched there, under the prologue's memory latency); it may write shared memory only past
 // C::LDS.

@@ -20,8 +20,10 @@
 
 // ---- pi_row_rgbx with alpha (procimg.h:592-630): c -> (c a + 255 (255 - a)) / 255 rounded, X = 255, in place. Four
 // pixels a thread (16 bytes at any pixel's alignment; a row's last pixels one by one); opaque pixels are left as they
-// are by the formula ((255 c) / 255 = c, X = 255 already), so four of them are not written back. Bound by HBM: 3072 x
-// 2048 with a translucent corner 13.6 -> 6 us against a read and a write of four bytes per thread.
+// are by the formula ((255 c) / 255 = c, X = 255 already), so four of them are not written back. Bound by HBM. us for
+// 3072 x 2048, one pixel a thread and every pixel written -> here, over 24 images in turn (4 images, which the caches
+// hold): opaque 17.6 -> 6.7 (13.2 -> 5.2), a sixteenth translucent 17.6 -> 7.4 (13.2 -> 5.8), all of it 17.7 -> 12.1
+// (13.2 -> 9.7).
 typedef unsigned img_u4 __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ uint32_t img_white(uint32_t v)
 {
@@ -111,11 +113,11 @@ __device__ __forceinline__ void img_bounds(const ImgGeom &g, int32_t i, float &c
     b = b < a ? a : b;
 }
 
-#define IMG_MT_MAX 24                       // taps per output up to a resample factor of 5 (mt = 2 (int)(2 f + 1) + 2)
+#define IMG_MT_MAX 24                       // taps per output for resample factors f < 5.5 (img_mt: 2 (int)(2 f + 1) + 2)
 #define IMG_XN (14 * IMG_BAND_P)            // outputs of a block's two axes: 28 columns, then 14 rows
 #define IMG_ON (IMG_XN + 14)
 #define IMG_RT 512                          // threads of k_img_resample
-#define IMG_SPAN 176                        // source columns of 28 outputs at that factor: 28 f + 4 f + 2 rounded up
+#define IMG_SPAN 176                        // source columns of 28 outputs: 27 f between centres + 4 f + 2 < 172.5
 
 // Tap tables (shared memory) of a block's outputs: columns x0 .. x0 + nx - 1 as outputs 0 .., rows y0 .. y0 + 13 as
 // outputs IMG_XN ..: every raw weight in parallel (the same float expression as the reference), then one thread per
@@ -317,8 +319,8 @@ extern "C" int eva_img_over_white(void *rgba, size_t stride, uint32_t w, uint32_
 {
     if (!rgba || !w || !h || stride < (size_t)w * 4 || (stride & 3) || ((uintptr_t)rgba & 3))
         return xt_fail("eva_img_over_white", "bad image (4-byte aligned rows of w RGBA pixels)");
-    hipLaunchKernelGGL(k_img_over_white, dim3((w + 255) / 256, (h + 3) / 4), dim3(256), 0, (hipStream_t)stream, (uint8_t *)rgba,
-                       stride, w, h);
+    hipLaunchKernelGGL(k_img_over_white, dim3((w + 255) / 256, (h + 3) / 4), dim3(256), 0, (hipStream_t)stream,
+                       (uint8_t *)rgba, stride, w, h);
     return xt_check("eva_img_over_white");
 }
 
@@ -417,7 +419,7 @@ static int img_rect(const char *what, const eva_pyr *p, uint32_t x0, uint32_t y0
     r.side = r.cw > r.ch ? r.cw : r.ch;
     r.S = S;
     if (r.side != S && img_mt(r.side, S) > IMG_MT_MAX)
-        return xt_fail(what, "rect more than 5x the model side on its level");
+        return xt_fail(what, "rect more than 5x the model side on its level");  // from 5.5x on
     return 0;
 }
 

@@ -143,7 +143,10 @@ k_ln(const uint16_t *__restrict__ x, const float *__restrict__ g, const float *_
 // k_pool: mean over tokens 1..1024 of each image: x fp16 [nb * 1025][1024] -> p fp32 [nb][1024]. Grid (nb, 8) of
 // 512 threads, 128 columns per block: thread (g, c) = (t >> 4, t & 15) sums tokens 1 + 32 g .. 32 g + 32 of columns
 // 8 c .. 8 c + 7 in token order, one 16-byte load per token; a column's 32 group sums then meet in group order
-// through shared memory, and the total is scaled by 1/1024.
+// through shared memory, and the total is scaled by 1/1024. Bound by HBM at 32 images, by the latency of a thread's few
+// loads in flight at one. The loop is unrolled whole, which the compiler turns into 8 loads and then a refill after each
+// use or two, 4 to 6 in flight (53 VGPRs; all 32 at once would take 128), where unrolling by 8 drained each 8 before the
+// next: 6.1 -> 5.4 us at 16 images, 4.36 -> 4.15 at one.
 __global__ void __launch_bounds__(512) k_pool(const uint16_t *__restrict__ x, float *__restrict__ p)
 {
     __shared__ __attribute__((aligned(16))) float red[32][128 + 4];
@@ -239,10 +242,11 @@ __global__ void __launch_bounds__(256) k_px_pembed(uint16_t *__restrict__ x, con
 // shared memory as well; then wave w forms the 16 x 16 scores' sums over k in [128 w, 128 w + 128) on the fp32 matrix
 // core (v_mfma_f32_16x16x4_f32: fp32 products of the fp16 y and the fp32 U, fp32 sums), its 128 x 16 slice of U held
 // in registers since before the rows arrived. Eight accumulators per wave take 16 products per score each, as many as a
-// lane's fma chain took before; the 64 partial sums of a score then meet in a fixed tree. Bound by HBM and L2 (x, hpos, U in, y out). The version before,
-// with U in 64 KB of shared memory and each score an fma chain and a butterfly over the wave (about 600 VALU
-// instructions and 64 KB of LDS reads per row, 64 rows per block), ran 47.1 us for 10368 rows and 95.7 for 41472;
-// this one 17.8 and 48 (3.7 TB/s over 180 MB). Scores against float64, rms: 1.64e-7 here, 1.64e-7 before.
+// lane's fma chain took before; the 64 partial sums of a score then meet in a fixed tree. Bound by HBM and L2 (x, hpos,
+// U in, y out). The version before, with U in 64 KB of shared memory and each score an fma chain and a butterfly over
+// the wave (about 600 VALU instructions and 64 KB of LDS reads per row, 64 rows per block), ran 47.1 us for 10368 rows
+// and 95.7 for 41472; this one 17.8 and 48 (3.7 TB/s over 180 MB). Scores against float64, rms: 1.64e-7 here, 1.64e-7
+// before.
 constexpr int PX_HLN_ROWS = 16;
 constexpr int PX_HLN_LD = XT_D + 8;  // halves per row of y in shared memory (rows start 4 banks apart)
 __global__ void __launch_bounds__(512) k_px_hln(const uint16_t *__restrict__ x, const float *__restrict__ g,

@@ -160,9 +160,9 @@ __global__ void __launch_bounds__(C::NT) k_px_res(const uint8_t *__restrict__ a8
 // k_px_fc1: h8 [rows][1024] x W1 [4736][1024] -> h = rs (gelu(acc + b1)), gelu(u) = u Phi(u) (exact normal CDF,
 // px_kernels.cu:228-231, by gelu_erf; rs may be NULL = 1), packed to m8 [rows][4736] E4M3 with 1x128 scales
 // ms [37][lds]. A wave's 128 columns are one scale block: each row's |max| meets in a 4-lane reduction (the tile is
-// transposed), the values are scaled in registers, parked in the wave's own LDS slice 64 columns at a time and stored 8 consecutive
-// bytes per lane (8 rows of 64 bytes per wave instruction). The second half of the last column tile lies past
-// unit 4736 and stores nothing.
+// transposed), the values are scaled in registers, parked in the wave's own LDS slice 64 columns at a time and stored 8
+// consecutive bytes per lane (8 rows of 64 bytes per wave instruction). 4736 units are 37 blocks of 128: with 256-column
+// tiles the second half of the last one lies past them and stores nothing, 128-column tiles end with them.
 // ---------------------------------------------------------------------------------------------------------------
 template <class C, bool RS>
 __global__ void __launch_bounds__(C::NT) k_px_fc1(const uint8_t *__restrict__ h8, const float *__restrict__ hs,
