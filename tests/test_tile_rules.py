@@ -4,6 +4,7 @@ are there for. CPU only."""
 import concurrent.futures
 import ctypes as C
 import os
+import re
 import shutil
 import subprocess
 
@@ -16,9 +17,11 @@ HIPCC = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
 pytestmark = pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
 
 # (source, the expression that calls its rule with a generic lambda f)
-RULES = {"res": ("layer.hip", "with_res_cfg(a, b, f)"), "qkv": ("layer.hip", "with_qkv_cfg(a, f)"),
+RULES = {"res": ("layer.hip", "with_res_cfg(a, b, 1, f)"), "qkv": ("layer.hip", "with_qkv_cfg(a, 1, f)"),
          "fc1": ("layer.hip", "with_fc1_cfg(a, f)"), "pe": ("layer.hip", "with_pe_cfg(a, f)"),
-         "px_fc1": ("px.hip", "with_px_fc1_cfg(a, f)"), "gemm": ("quant.hip", "with_gemm_cfg(a, b, f)")}
+         "px_fc1": ("px.hip", "with_px_fc1_cfg(a, 1, f)"), "gemm": ("quant.hip", "with_gemm_cfg(a, b, f)"),
+         "res_2": ("layer.hip", "with_res_cfg(a, b, 2, f)"), "qkv_2": ("layer.hip", "with_qkv_cfg(a, 2, f)"),
+         "px_fc1_2": ("px.hip", "with_px_fc1_cfg(a, 2, f)")}
 
 
 @pytest.fixture(scope="module")
@@ -72,6 +75,22 @@ def test_both_sides_of_every_limit(tile):
     assert _limits(tile, "px_fc1", 20000) == [12288]
     assert [tile("qkv", 1025 * nb) for nb in (1, 2, 3, 5, 6, 7, 8, 16, 32)] == [MID, MID, BIG, BIG, MID, BIG, BIG, BIG, BIG]
     assert [tile("pe", r) for r in (1024, 2048, 2049, 3072)] == [(64, 64), (64, 64), MID, MID]
+
+
+def test_two_lanes(tile):
+    """Beside an engine's other lane the tiles that only win alone on the chip (128 x 128 from 4353 rows on, qkv's for a
+    short second round, PixAI fc1's) are not taken: batches of 10 to 14 images lost 2 to 5% with them."""
+    for k in (G.D, G.HIDP, G.PXH):
+        assert _limits(tile, "res_2", 42000, k) == [4096, 4352], k
+        assert [tile("res_2", r, k) for r in (4096, 4100, 5125, 16400)] == [SML, MID, BIG, BIG]
+    assert _limits(tile, "qkv_2", 42000) == [2688] and tile("qkv_2", 1025) == MID
+    assert _limits(tile, "px_fc1_2", 42000) == [] and tile("px_fc1_2", 10368) == BIG
+    used = {"engine.cpp": ("xt_qkv", "xt_oproj", "xt_fc2"), "px_engine.cpp": ("xt_px_proj", "xt_px_fc1", "xt_px_fc2")}
+    for src, names in used.items():                           # the engines call the launchers that take their lanes
+        text = open(os.path.join(CSRC, src)).read()
+        for n in names:
+            assert n + "(" in text, (src, n)
+            assert not re.search(n.replace("xt_px_", "px_k_").replace("xt_", "eva_k_") + r"(_sp)?\(", text), (src, n)
 
 
 def test_partial_row_tiles_cover_every_tile(tile):

@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "xt_abi.h"
+#include "xt_launch.h"
 #include "xt_stream.h"
 #include "xtag_eva.h"
 
@@ -185,25 +186,25 @@ static int ev_forward(eva *e, hipStream_t fst)
 {
     eva_impl *E = e->impl;
     void *st = (void *)fst;
-    const int M = (int)E->cM, lds = (int)E->cMp, nb = (int)E->cnb;
+    const int M = (int)E->cM, lds = (int)E->cMp, nb = (int)E->cnb, nl = (int)E->nl;
 
     EV_OP(eva_k_pe(E->in, E->pe, E->pos, E->x, nb, st), 0);
     for (int i = 0; i < EVA_NL; i++) {
         const Layer &L = E->L[i];
         const bool sp = E->flags & EVA_SPARSE24;
         EV_OP(eva_k_ln(E->x, L.ln1w, L.ln1b, E->h8, E->sh, M, lds, st), 1);
-        if (sp) EV_OP(eva_k_qkv_sp(E->h8, E->sh, lds, L.vqkv, L.xqkv, L.sqkv, E->cs, E->q, E->k, E->vt, M, st), 2);
-        else EV_OP(eva_k_qkv(E->h8, E->sh, lds, L.wqkv, L.sqkv, E->cs, E->q, E->k, E->vt, M, st), 2);
+        if (sp) EV_OP(xt_qkv(E->h8, E->sh, lds, L.vqkv, L.xqkv, L.sqkv, E->cs, E->q, E->k, E->vt, M, nl, st), 2);
+        else EV_OP(xt_qkv(E->h8, E->sh, lds, L.wqkv, NULL, L.sqkv, E->cs, E->q, E->k, E->vt, M, nl, st), 2);
         EV_OP(eva_k_flash(E->q, E->k, E->vt, E->h8, E->sh, lds, nb, NULL, st), 3);
-        if (sp) EV_OP(eva_k_oproj_sp(E->h8, E->sh, lds, L.vo, L.xo, L.so, E->x, M, st), 4);
-        else EV_OP(eva_k_oproj(E->h8, E->sh, lds, L.wo, L.so, E->x, M, st), 4);
+        if (sp) EV_OP(xt_oproj(E->h8, E->sh, lds, L.vo, L.xo, L.so, E->x, M, nl, st), 4);
+        else EV_OP(xt_oproj(E->h8, E->sh, lds, L.wo, NULL, L.so, E->x, M, nl, st), 4);
         EV_OP(eva_k_ln(E->x, L.ln2w, L.ln2b, E->h8, E->sh, M, lds, st), 5);
         if (sp && L.rs) EV_OP(eva_k_fc1_rs_sp(E->h8, E->sh, lds, L.v12, L.x12, L.s12, E->m8, E->sm, E->stat, L.rs, M, st), 6);
         else if (sp) EV_OP(eva_k_fc1_sp(E->h8, E->sh, lds, L.v12, L.x12, L.s12, E->m8, E->sm, E->stat, M, st), 6);
         else if (L.rs) EV_OP(eva_k_fc1_rs(E->h8, E->sh, lds, L.w12, L.s12, E->m8, E->sm, E->stat, L.rs, M, st), 6);
         else EV_OP(eva_k_fc1(E->h8, E->sh, lds, L.w12, L.s12, E->m8, E->sm, E->stat, M, st), 6);
-        if (sp) EV_OP(eva_k_fc2_sp(E->m8, E->sm, lds, L.v2, L.x2, L.s2, E->stat, L.cn, L.dn, E->x, M, st), 7);
-        else EV_OP(eva_k_fc2(E->m8, E->sm, lds, L.w2, L.s2, E->stat, L.cn, L.dn, E->x, M, st), 7);
+        if (sp) EV_OP(xt_fc2(E->m8, E->sm, lds, L.v2, L.x2, L.s2, E->stat, L.cn, L.dn, E->x, M, nl, st), 7);
+        else EV_OP(xt_fc2(E->m8, E->sm, lds, L.w2, NULL, L.s2, E->stat, L.cn, L.dn, E->x, M, nl, st), 7);
     }
     EV_CK(eva_k_pool(E->x, E->pool, nb, st));
     EV_CK(eva_k_lnh(E->pool, E->fnw, E->fnb, E->pn, E->pq, E->ps, nb, nb, st));

@@ -545,12 +545,13 @@ __global__ void __launch_bounds__(C::NT) k_pe(const uint16_t *__restrict__ in, c
 // ---------------------------------------------------------------------------------------------------------------
 // qkv's tiles: 128 x 128 while one round of two blocks per CU holds them (rows <= 2688: 17.2 -> 8.4 us at 1025 rows,
 // 18.5 -> 12.7 at 2050), and where 256 x 256 tiles would run a second round less than a quarter full (6150 rows: 34.3
-// -> 30.0 us); 256 x 256 elsewhere (20.6 against 22.1 us at 4100, 34.8 against 38.8 at 8200).
+// -> 30.0 us; not beside an engine's other lane, which takes the CUs of that round: 6725 -> 6950 us a batch of 12
+// images); 256 x 256 elsewhere (20.6 against 22.1 us at 4100, 34.8 against 38.8 at 8200).
 template <class F>
-static void with_qkv_cfg(int rows, F f)
+static void with_qkv_cfg(int rows, int lanes, F f)
 {
     const unsigned big = layer_grid<LayerCfg>(rows, 3 * XT_D);
-    if (rows <= 2688 || (big > 256 && big <= 320)) f(LayerMid{});
+    if (rows <= 2688 || (lanes == 1 && big > 256 && big <= 320)) f(LayerMid{});
     else f(LayerCfg{});
 }
 
@@ -567,12 +568,12 @@ static void with_fc1_cfg(int rows, F f)
 
 template <bool SP>
 static int qkv_launch(const char *what, const void *h8, const float *hs, int lds, const void *w, const void *wx,
-                      const float *ws, const float *cs, void *q, void *k, void *vt, int rows, void *stream)
+                      const float *ws, const float *cs, void *q, void *k, void *vt, int rows, int lanes, void *stream)
 {
     if (layer_rows_ok(what, rows, lds)) return -1;
     if (rows % XT_T) return xt_fail(what, "rows must be nb * 1025");
     if (!XT_ALIGNED(h8) || !XT_ALIGNED(w) || (SP && !wx)) return xt_fail(what, "h8 and w must be 16-byte aligned");
-    with_qkv_cfg(rows, [&](auto c) {
+    with_qkv_cfg(rows, lanes, [&](auto c) {
         using C = decltype(c);
         hipLaunchKernelGGL((k_qkv<C, SP>), dim3(layer_grid<C>(rows, 3 * XT_D)), dim3(C::NT), 0, (hipStream_t)stream,
                            (const uint8_t *)h8, hs, lds, (const uint8_t *)w, (const uint32_t *)wx, ws, cs,
@@ -583,11 +584,11 @@ static int qkv_launch(const char *what, const void *h8, const float *hs, int lds
 
 template <bool SP>
 static int oproj_launch(const char *what, const void *a8, const float *as, int lds, const void *w, const void *wx,
-                        const float *ws, void *x, int rows, void *stream)
+                        const float *ws, void *x, int rows, int lanes, void *stream)
 {
     if (layer_rows_ok(what, rows, lds)) return -1;
     if (!XT_ALIGNED(a8) || !XT_ALIGNED(w) || (SP && !wx)) return xt_fail(what, "a8 and w must be 16-byte aligned");
-    with_res_cfg(rows, XT_D, [&](auto c) {
+    with_res_cfg(rows, XT_D, lanes, [&](auto c) {
         using C = decltype(c);
         hipLaunchKernelGGL((k_oproj<C, SP>), dim3(layer_grid<C>(rows, XT_D)), dim3(C::NT), 0, (hipStream_t)stream,
                            (const uint8_t *)a8, as, lds, (const uint8_t *)w, (const uint32_t *)wx, ws, (uint16_t *)x,
@@ -619,11 +620,11 @@ static int fc1_launch(const char *what, const void *h8, const float *hs, int lds
 template <bool SP>
 static int fc2_launch(const char *what, const void *m8, const float *ms, int lds, const void *w, const void *wx,
                       const float *ws, const float *stat, const float *cn, const float *dn, void *x, int rows,
-                      void *stream)
+                      int lanes, void *stream)
 {
     if (layer_rows_ok(what, rows, lds)) return -1;
     if (!XT_ALIGNED(m8) || !XT_ALIGNED(w) || (SP && !wx)) return xt_fail(what, "m8 and w must be 16-byte aligned");
-    with_res_cfg(rows, XT_HIDP, [&](auto c) {
+    with_res_cfg(rows, XT_HIDP, lanes, [&](auto c) {
         using C = decltype(c);
         hipLaunchKernelGGL((k_fc2<C, SP>), dim3(layer_grid<C>(rows, XT_D)), dim3(C::NT), 0, (hipStream_t)stream,
                            (const uint8_t *)m8, ms, lds, (const uint8_t *)w, (const uint32_t *)wx, ws, stat, cn, dn,
@@ -632,16 +633,37 @@ static int fc2_launch(const char *what, const void *m8, const float *ms, int lds
     return xt_check(what);
 }
 
+int xt_qkv(const void *h8, const float *hs, int lds, const void *w, const void *wx, const float *ws, const float *cs,
+           void *q, void *k, void *vt, int rows, int lanes, void *stream)
+{
+    return wx ? qkv_launch<true>("eva_k_qkv_sp", h8, hs, lds, w, wx, ws, cs, q, k, vt, rows, lanes, stream)
+              : qkv_launch<false>("eva_k_qkv", h8, hs, lds, w, wx, ws, cs, q, k, vt, rows, lanes, stream);
+}
+
+int xt_oproj(const void *a8, const float *as, int lds, const void *w, const void *wx, const float *ws, void *x, int rows,
+             int lanes, void *stream)
+{
+    return wx ? oproj_launch<true>("eva_k_oproj_sp", a8, as, lds, w, wx, ws, x, rows, lanes, stream)
+              : oproj_launch<false>("eva_k_oproj", a8, as, lds, w, wx, ws, x, rows, lanes, stream);
+}
+
+int xt_fc2(const void *m8, const float *ms, int lds, const void *w, const void *wx, const float *ws, const float *stat,
+           const float *cn, const float *dn, void *x, int rows, int lanes, void *stream)
+{
+    return wx ? fc2_launch<true>("eva_k_fc2_sp", m8, ms, lds, w, wx, ws, stat, cn, dn, x, rows, lanes, stream)
+              : fc2_launch<false>("eva_k_fc2", m8, ms, lds, w, wx, ws, stat, cn, dn, x, rows, lanes, stream);
+}
+
 extern "C" int eva_k_qkv(const void *h8, const float *hs, int lds, const void *w, const float *ws, const float *cs,
                          void *q, void *k, void *vt, int rows, void *stream)
 {
-    return qkv_launch<false>("eva_k_qkv", h8, hs, lds, w, nullptr, ws, cs, q, k, vt, rows, stream);
+    return qkv_launch<false>("eva_k_qkv", h8, hs, lds, w, nullptr, ws, cs, q, k, vt, rows, 1, stream);
 }
 
 extern "C" int eva_k_oproj(const void *a8, const float *as, int lds, const void *w, const float *ws, void *x, int rows,
                            void *stream)
 {
-    return oproj_launch<false>("eva_k_oproj", a8, as, lds, w, nullptr, ws, x, rows, stream);
+    return oproj_launch<false>("eva_k_oproj", a8, as, lds, w, nullptr, ws, x, rows, 1, stream);
 }
 
 extern "C" int eva_k_fc1(const void *h8, const float *hs, int lds, const void *w, const float *ws, void *m8, float *ms,
@@ -660,19 +682,19 @@ extern "C" int eva_k_fc1_rs(const void *h8, const float *hs, int lds, const void
 extern "C" int eva_k_fc2(const void *m8, const float *ms, int lds, const void *w, const float *ws, const float *stat,
                          const float *cn, const float *dn, void *x, int rows, void *stream)
 {
-    return fc2_launch<false>("eva_k_fc2", m8, ms, lds, w, nullptr, ws, stat, cn, dn, x, rows, stream);
+    return fc2_launch<false>("eva_k_fc2", m8, ms, lds, w, nullptr, ws, stat, cn, dn, x, rows, 1, stream);
 }
 
 extern "C" int eva_k_qkv_sp(const void *h8, const float *hs, int lds, const void *vals, const void *idx,
                             const float *ws, const float *cs, void *q, void *k, void *vt, int rows, void *stream)
 {
-    return qkv_launch<true>("eva_k_qkv_sp", h8, hs, lds, vals, idx, ws, cs, q, k, vt, rows, stream);
+    return qkv_launch<true>("eva_k_qkv_sp", h8, hs, lds, vals, idx, ws, cs, q, k, vt, rows, 1, stream);
 }
 
 extern "C" int eva_k_oproj_sp(const void *a8, const float *as, int lds, const void *vals, const void *idx,
                               const float *ws, void *x, int rows, void *stream)
 {
-    return oproj_launch<true>("eva_k_oproj_sp", a8, as, lds, vals, idx, ws, x, rows, stream);
+    return oproj_launch<true>("eva_k_oproj_sp", a8, as, lds, vals, idx, ws, x, rows, 1, stream);
 }
 
 extern "C" int eva_k_fc1_sp(const void *h8, const float *hs, int lds, const void *vals, const void *idx,
@@ -693,7 +715,7 @@ extern "C" int eva_k_fc2_sp(const void *m8, const float *ms, int lds, const void
                             const float *ws, const float *stat, const float *cn, const float *dn, void *x, int rows,
                             void *stream)
 {
-    return fc2_launch<true>("eva_k_fc2_sp", m8, ms, lds, vals, idx, ws, stat, cn, dn, x, rows, stream);
+    return fc2_launch<true>("eva_k_fc2_sp", m8, ms, lds, vals, idx, ws, stat, cn, dn, x, rows, 1, stream);
 }
 
 extern "C" int eva_k_head(const void *pq, const float *ps, int lds, const void *w, const float *ws, int ldw,

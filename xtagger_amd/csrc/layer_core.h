@@ -4,6 +4,7 @@
 #pragma once
 #include "gemm_core.h"
 #include "xt_abi.h"
+#include "xt_launch.h"
 
 typedef BsCfg<256, 256, 4, 2, 2> LayerCfg;  // 8 waves of 64 x 128: two heads (qkv) or 64 SwiGLU units (fc1) per wave
 // Smaller tiles for grids that LayerCfg would leave mostly idle (with_res_cfg, and qkv's and fc1's own rules). Every
@@ -152,12 +153,18 @@ static inline unsigned layer_grid(int rows, int N)
 //    the rounds exactly and a partial row tile follows): 18.3 -> 16.9 at 8200, 31.9 -> 28.2 at 16400, 37.1 -> 34.5
 //    at 20736, 52.2 -> 46.9 at 32800 (a last round fuller than that: 18.9 against 19.3 at 10250, 44.0 against 48.9 at
 //    31104).
+// Those are calls alone on the chip. Beside an engine's other lane, whose kernels take the CUs that a grid leaves idle,
+// the 128 x 128 tiles' operand traffic costs more than they save: us per batch, the limits above (and qkv's) -> 256 x 256
+// from 4353 rows a lane on: 5950 -> 5640 at 10 images, 7015 -> 6750 at 12, 7750 -> 7620 at 14, the same within 1% from 16
+// to 64 (PixAI's proj: 30340 -> 30120 at 8). At 4100 rows 128 x 128 stays: 4300 against 4393 at 7 images, 4806 against
+// 4839 at 8.
 template <class F>
-static inline void with_res_cfg(int rows, int K, F f)
+static inline void with_res_cfg(int rows, int K, int lanes, F f)
 {
     const int tail = rows / LayerCfg::BM * (XT_D / LayerCfg::BN) % 256;  // whole 256 x 256 tiles of the last round
     if (rows <= 4096) f(LayerSml{});
-    else if (rows <= 8192 || (K <= XT_D && tail <= 128 && (tail || rows % LayerCfg::BM))) f(LayerMid{});
+    else if (lanes > 1 ? rows <= 4352 : rows <= 8192 || (K <= XT_D && tail <= 128 && (tail || rows % LayerCfg::BM)))
+        f(LayerMid{});
     else f(LayerCfg{});
 }
 

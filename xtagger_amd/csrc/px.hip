@@ -258,11 +258,11 @@ extern "C" int px_k_qkv(const void *h8, const float *hs, int lds, const void *w,
 
 template <int K>
 static int px_res_launch(const char *what, const void *a8, const float *as, int lds, const void *w, const float *ws,
-                         const float *bias, void *x, int rows, void *stream)
+                         const float *bias, void *x, int rows, int lanes, void *stream)
 {
     if (layer_rows_ok(what, rows, lds)) return -1;
     if (!XT_ALIGNED(a8) || !XT_ALIGNED(w)) return xt_fail(what, "a8 and w must be 16-byte aligned");
-    with_res_cfg(rows, K, [&](auto c) {
+    with_res_cfg(rows, K, lanes, [&](auto c) {
         using C = decltype(c);
         hipLaunchKernelGGL((k_px_res<C, K>), dim3(layer_grid<C>(rows, XT_D)), dim3(C::NT), 0, (hipStream_t)stream,
                            (const uint8_t *)a8, as, lds, (const uint8_t *)w, ws, bias, (uint16_t *)x, rows);
@@ -270,36 +270,49 @@ static int px_res_launch(const char *what, const void *a8, const float *as, int 
     return xt_check(what);
 }
 
+int xt_px_proj(const void *a8, const float *as, int lds, const void *w, const float *ws, const float *bias, void *x,
+               int rows, int lanes, void *stream)
+{
+    return px_res_launch<XT_D>("px_k_proj", a8, as, lds, w, ws, bias, x, rows, lanes, stream);
+}
+
+int xt_px_fc2(const void *m8, const float *ms, int lds, const void *w, const float *ws, const float *bias, void *x,
+              int rows, int lanes, void *stream)
+{
+    return px_res_launch<PX_HID>("px_k_fc2", m8, ms, lds, w, ws, bias, x, rows, lanes, stream);
+}
+
 extern "C" int px_k_proj(const void *a8, const float *as, int lds, const void *w, const float *ws, const float *bias,
                          void *x, int rows, void *stream)
 {
-    return px_res_launch<XT_D>("px_k_proj", a8, as, lds, w, ws, bias, x, rows, stream);
+    return xt_px_proj(a8, as, lds, w, ws, bias, x, rows, 1, stream);
 }
 
 extern "C" int px_k_fc2(const void *m8, const float *ms, int lds, const void *w, const float *ws, const float *bias,
                         void *x, int rows, void *stream)
 {
-    return px_res_launch<PX_HID>("px_k_fc2", m8, ms, lds, w, ws, bias, x, rows, stream);
+    return xt_px_fc2(m8, ms, lds, w, ws, bias, x, rows, 1, stream);
 }
 
 // k_px_fc1's tiles: 128 x 128 (4 waves of 32 x 128, two blocks per CU) up to 12288 rows: one block's GELU and packing
 // runs beside the other's main loop, and the last round wastes less (48.0 -> 41.4 us at 5184 rows, 85.2 -> 77.0 at
-// 10368); with more rounds 256 x 256 is as good or better (111 against 114 at 15552, 290 against 292 at 41472).
+// 10368); with more rounds 256 x 256 is as good or better (111 against 114 at 15552, 290 against 292 at 41472), and so
+// it is beside an engine's other lane, which covers them too (a batch of 6 images 23740 -> 23540 us, of 4 the same).
 typedef BsCfg<128, 128, 4, 1, 2> PxFc1Mid;
 template <class F>
-static void with_px_fc1_cfg(int rows, F f)
+static void with_px_fc1_cfg(int rows, int lanes, F f)
 {
-    if (rows <= 12288) f(PxFc1Mid{});
+    if (lanes == 1 && rows <= 12288) f(PxFc1Mid{});
     else f(LayerCfg{});
 }
 
-extern "C" int px_k_fc1(const void *h8, const float *hs, int lds, const void *w, const float *ws, const float *bias,
-                        const float *rs, void *m8, float *ms, int rows, void *stream)
+int xt_px_fc1(const void *h8, const float *hs, int lds, const void *w, const float *ws, const float *bias,
+              const float *rs, void *m8, float *ms, int rows, int lanes, void *stream)
 {
     if (layer_rows_ok("px_k_fc1", rows, lds)) return -1;
     if (!XT_ALIGNED(h8) || !XT_ALIGNED(w) || ((uintptr_t)m8 & 7))
         return xt_fail("px_k_fc1", "h8 and w must be 16-byte aligned, m8 8-byte aligned");
-    with_px_fc1_cfg(rows, [&](auto c) {
+    with_px_fc1_cfg(rows, lanes, [&](auto c) {
         using C = decltype(c);
         const dim3 grid(layer_grid<C>(rows, PX_HID));
         if (rs)  // the multiply only where rs is given
@@ -310,6 +323,12 @@ extern "C" int px_k_fc1(const void *h8, const float *hs, int lds, const void *w,
                                lds, (const uint8_t *)w, ws, bias, rs, (uint8_t *)m8, ms, rows);
     });
     return xt_check("px_k_fc1");
+}
+
+extern "C" int px_k_fc1(const void *h8, const float *hs, int lds, const void *w, const float *ws, const float *bias,
+                        const float *rs, void *m8, float *ms, int rows, void *stream)
+{
+    return xt_px_fc1(h8, hs, lds, w, ws, bias, rs, m8, ms, rows, 1, stream);
 }
 
 // ---------------------------------------------------------------------------------------------------------------

@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "xt_abi.h"
+#include "xt_launch.h"
 #include "xt_stream.h"
 #include "xtag_eva.h"
 
@@ -165,7 +166,7 @@ static int px_forward(px *p, hipStream_t fst)
 {
     px_impl *E = p->impl;
     void *st = (void *)fst;
-    const int M = (int)E->cM, nb = (int)E->cnb;
+    const int M = (int)E->cM, nb = (int)E->cnb, nl = (int)E->nl;
 
     PX_CK(px_k_pe(E->in, E->pe, E->x, M, st));
     PX_CK(px_k_pembed(E->x, E->pos, PX_T, E->lnpw, E->lnpb, M, st));
@@ -176,10 +177,10 @@ static int px_forward(px *p, hipStream_t fst)
         PX_CK(eva_k_ln(E->x, L.ln1w, L.ln1b, E->h8, E->sh, M, M, st));
         PX_CK(px_k_qkv(E->h8, E->sh, M, L.wqkv, L.sqkv, L.bqkv, glob ? E->csg : E->csw, Ls, E->q, E->k, E->vt, M, st));
         PX_CK(eva_k_flash_seq(E->q, E->k, E->vt, E->o8, E->so8, M, M / Ls, Ls, Ls, NULL, st));
-        PX_CK(px_k_proj(E->o8, E->so8, M, L.wo, L.so, L.bo, E->x, M, st));
+        PX_CK(xt_px_proj(E->o8, E->so8, M, L.wo, L.so, L.bo, E->x, M, nl, st));
         PX_CK(eva_k_ln(E->x, L.ln2w, L.ln2b, E->h8, E->sh, M, M, st));
-        PX_CK(px_k_fc1(E->h8, E->sh, M, L.w1, L.s1, L.b1, L.rs_fc1, E->m8, E->sm, M, st));
-        PX_CK(px_k_fc2(E->m8, E->sm, M, L.w2, L.s2, L.b2, E->x, M, st));
+        PX_CK(xt_px_fc1(E->h8, E->sh, M, L.w1, L.s1, L.b1, L.rs_fc1, E->m8, E->sm, M, nl, st));
+        PX_CK(xt_px_fc2(E->m8, E->sm, M, L.w2, L.s2, L.b2, E->x, M, nl, st));
     }
     PX_CK(px_k_hln(E->x, E->hnw, E->hnb, E->hpos, PX_T, E->U, E->y, E->s, M, st));
     PX_CK(px_k_hstat(E->s, E->stat, nb, PX_T, st));
