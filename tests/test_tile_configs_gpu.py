@@ -195,7 +195,8 @@ def test_hln_ragged_rows(dev, xt, orc, rows):
 @pytest.mark.parametrize("sparse", [False, True])
 @pytest.mark.parametrize("M,N,K,off,pad", [(1, 64, 128, 0, 0), (65, 207, 256, 1, 3), (1025, 3071, 1024, 0, 1),
                                             (1025, 1024, 512, 3, 0), (2050, 3088, 128, 0, 0), (4100, 3072, 256, 5, 2),
-                                            (8200, 2000, 128, 0, 8), (1025, 13461, 128, 0, 0)])
+                                            (8200, 2000, 128, 0, 8), (1025, 13461, 128, 0, 0), (4100, 3072, 256, 0, 0),
+                                            (3000, 4096, 2048, 8, 8), (2049, 3072, 256, 16, 16), (2050, 3088, 256, 3, 1)])
 def test_gemm_any_alignment_and_tile(dev, xt, M, N, K, off, pad, sparse):
     """C at any element offset and row stride, N ragged: the same bits as the fp32 output of the aligned call row by
     row (in pieces of 64 rows: the smallest tiles), bf16 rounded to nearest even, nothing written outside C."""

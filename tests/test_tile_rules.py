@@ -19,19 +19,21 @@ pytestmark = pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not ava
 # (source, the expression that calls its rule with a generic lambda f)
 RULES = {"res": ("layer.hip", "with_res_cfg(a, b, 1, f)"), "qkv": ("layer.hip", "with_qkv_cfg(a, 1, f)"),
          "fc1": ("layer.hip", "with_fc1_cfg(a, f)"), "pe": ("layer.hip", "with_pe_cfg(a, f)"),
-         "px_fc1": ("px.hip", "with_px_fc1_cfg(a, 1, f)"), "gemm": ("quant.hip", "with_gemm_cfg(a, b, f)"),
+         "px_fc1": ("px.hip", "with_px_fc1_cfg(a, 1, f)"),
+         "gemm": ("quant.hip", "with_gemm_cfg<false>(a, b, c, out, f)"),
+         "gemm_sp": ("quant.hip", "with_gemm_cfg<true>(a, b, c, out, f)"),
          "res_2": ("layer.hip", "with_res_cfg(a, b, 2, f)"), "qkv_2": ("layer.hip", "with_qkv_cfg(a, 2, f)"),
          "px_fc1_2": ("px.hip", "with_px_fc1_cfg(a, 2, f)")}
 
 
 @pytest.fixture(scope="module")
 def tile(tmp_path_factory):
-    """tile(rule, a, b=0) -> (BM, BN)"""
+    """tile(rule, a, b=0, c=0, out=2) -> (BM, BN, waves)"""
     d = tmp_path_factory.mktemp("rules")
 
     def build(src):
-        body = "".join(f'extern "C" int rule_{k}(int a, int b) {{ int t = 0; auto f = [&](auto c) {{ using T = '
-                       f'decltype(c); t = 1000 * T::BM + T::BN; }}; {e}; return t; }}\n'
+        body = "".join(f'extern "C" int rule_{k}(int a, int b, int c, int out) {{ int t = 0; auto f = [&](auto x) {{ '
+                       f'using T = decltype(x); t = (T::BM * 1000 + T::BN) * 1000 + T::NW; }}; {e}; return t; }}\n'
                        for k, (s, e) in RULES.items() if s == src)
         f = d / ("q_" + src)
         f.write_text(f'#include "{os.path.join(CSRC, src)}"\n{body}')
@@ -45,7 +47,12 @@ def tile(tmp_path_factory):
 
     with concurrent.futures.ThreadPoolExecutor(3) as ex:
         libs = dict(ex.map(build, sorted({s for s, _ in RULES.values()})))
-    return lambda rule, a, b=0: divmod(getattr(libs[RULES[rule][0]], "rule_" + rule)(a, b), 1000)
+
+    def tile(rule, a, b=0, c=0, out=2):
+        t = getattr(libs[RULES[rule][0]], "rule_" + rule)(a, b, c, out)
+        return t // 1000000, t // 1000 % 1000, t % 1000
+
+    return tile
 
 
 def _limits(tile, rule, hi, *args):
@@ -54,7 +61,7 @@ def _limits(tile, rule, hi, *args):
     return [r for r in range(1, hi) if t[r - 1] != t[r]]
 
 
-SML, MID, BIG = (64, 128), (128, 128), (256, 256)
+SML, MID, BIG = (64, 128, 4), (128, 128, 8), (256, 256, 8)
 
 
 def test_both_sides_of_every_limit(tile):
@@ -74,7 +81,7 @@ def test_both_sides_of_every_limit(tile):
     assert _limits(tile, "fc1", 20000) == [1408] and {1408, 1409} <= set(G.RES_ROWS)
     assert _limits(tile, "px_fc1", 20000) == [12288]
     assert [tile("qkv", 1025 * nb) for nb in (1, 2, 3, 5, 6, 7, 8, 16, 32)] == [MID, MID, BIG, BIG, MID, BIG, BIG, BIG, BIG]
-    assert [tile("pe", r) for r in (1024, 2048, 2049, 3072)] == [(64, 64), (64, 64), MID, MID]
+    assert [tile("pe", r) for r in (1024, 2048, 2049, 3072)] == [(64, 64, 4), (64, 64, 4), MID, MID]
 
 
 def test_two_lanes(tile):
@@ -96,11 +103,32 @@ def test_two_lanes(tile):
 def test_partial_row_tiles_cover_every_tile(tile):
     for k in (G.D, G.HIDP):
         assert [{tile("res", b + t, k) for t in G.TAILS} for b in G.TAIL_BASES[1:]] == [{SML}, {MID}, {BIG}], k
-    assert [{tile("fc1", b + t) for t in G.TAILS} for b in G.TAIL_BASES] == [{(128, 256)}, {BIG}, {BIG}, {BIG}]
+    assert [{tile("fc1", b + t) for t in G.TAILS} for b in G.TAIL_BASES] == [{(128, 256, 16)}, {BIG}, {BIG}, {BIG}]
 
 
 def test_gemm_shapes_cover_every_tile(tile):
     shapes = next(m for m in G.test_gemm_any_alignment_and_tile.pytestmark if "M,N" in m.args[0]).args[1]
-    for sparse in (False, True):
-        got = {tile("gemm", M, (N + 15) // 16 * 16 if sparse else N) for M, N, *_ in shapes}
-        assert got == {(64, 64), SML, MID, BIG}, got
+    narrow, wide = {(64, 64, 4), SML, MID}, {(128, 128, 4), BIG}
+    for rule in ("gemm", "gemm_sp"):
+        got = {0: set(), 1: set(), 2: set()}                  # by what is stored: bf16, fp32, bf16 to an aligned C
+        for M, N, K, off, pad in shapes:
+            n = (N + 15) // 16 * 16 if rule == "gemm_sp" else N
+            out = 2 if (n | n + pad | off) % 8 == 0 else 0
+            for o in (out, 1):
+                got[o].add(tile(rule, M, n, K, o))
+        assert got[1] == narrow | wide, (rule, got[1])
+        assert got[2] >= wide and got[0] >= {BIG, MID} and got[0] | got[2] == narrow | wide, (rule, got)
+        assert (128, 128, 4) not in got[0]
+
+
+def test_gemm_limits(tile):
+    """both sides of the rule's lines: rounds of 512 blocks (128 x 128) and 256 blocks (256 x 256), and K"""
+    wide = (128, 128, 4)
+    for args, want in {(3000, 4096, 512): wide, (3000, 4096, 2048): BIG, (3584, 3584, 128): BIG, (4000, 4000, 128): BIG,
+                       (4100, 4000, 128): MID, (8100, 3000, 2048): wide, (8200, 3072, 2047): MID, (8200, 3072, 2048): BIG,
+                       (2050, 3072, 3072): wide, (8200, 1024, 1024): MID, (3200, 8000, 128): BIG}.items():
+        assert tile("gemm", *args) == want, args
+    for args, want in {(3000, 4096, 128): wide, (3000, 4096, 2048): MID, (3584, 3584, 128): BIG, (2050, 3072, 128): wide,
+                       (2050, 3072, 256): MID, (8200, 3072, 3072): MID}.items():
+        assert tile("gemm_sp", *args) == want, args
+    assert tile("gemm_sp", 2050, 3072, 896, 1) == wide and tile("gemm_sp", 2050, 3072, 1024, 1) == MID

@@ -1,6 +1,8 @@
 // quant.hip - E4M3 packing with per-block fp32 scales (activations 1x128, weights 128x128) and the standalone
 // block-scaled GEMM. Reference roles: q2 / st4 / st8h (src/engine/kern_common.cuh:97-128) for activations,
 // fp8() (src/tools/export_eva.py:64-66) for weights, gemm8 (kern_common.cuh:271-356) for the GEMM.
+#include <type_traits>
+
 #include "layer_core.h"
 
 // ---- activations: x [M][ldx] (bf16, fp32 or fp16) -> q [M][ldq] E4M3, s [K/128][lds] ----
@@ -114,10 +116,13 @@ __global__ void __launch_bounds__(256) k_scale_bits(uint32_t first, uint32_t cou
 // bf16: each wave parks its rows x 64 (or 32) fp32 of its tile in its own LDS slice (padded rows, conflict-free), then
 // every lane rounds 8 consecutive columns to bf16 (RNE) and writes them with one 16-byte store, whatever the row's
 // alignment (the hardware takes 16-byte stores at any element address; two-byte stores for an odd ldc or N, as before,
-// took 242 us for 8200 x 13461 x 1024). fp32 stores 16 bytes straight from the accumulators. Columns of a store that
-// reaches past N go one by one.
+// took 242 us for 8200 x 13461 x 1024). Columns of a store that reaches past N go one by one. In the tiles of
+// 64-row waves an aligned C (ldc and N multiples of 8, 16-byte aligned) has a kernel of its own that stores through a
+// descriptor ending at row M, without 64-bit addresses and row compares: 4100 x 13456 x 1024 77.9 -> 76.0 us, 8200 x 5632
+// x 1024 58.7 -> 57.6 (with 32-row waves slower: 4100 x 2048 x 256 8.9 -> 9.5). fp32 stores 16 bytes straight from the
+// accumulators.
 // SP: W holds the 2:4 values and WX the indices of the pack24 layout (bs_mainloop_sp); otherwise W is dense, WX unused.
-template <class C, int OUT, bool SP>  // OUT 0: bf16, 1: fp32
+template <class C, int OUT, bool SP>  // OUT 0: bf16, 1: fp32, 2: bf16 of an aligned C
 __global__ void __launch_bounds__(C::NT) k_gemm(const uint8_t *__restrict__ A, int lda, const float *__restrict__ sa,
                                                int lds, const uint8_t *__restrict__ W, const uint32_t *__restrict__ WX,
                                                const float *__restrict__ sw, void *__restrict__ Cp, int ldc, int M,
@@ -140,7 +145,7 @@ __global__ void __launch_bounds__(C::NT) k_gemm(const uint8_t *__restrict__ A, i
 #pragma unroll
             for (int j = 0; j < C::TN; j++) acc[i][j] = accT[j][i];
     } else {
-        bs_mainloop<C, BsNoPre, C::TM == 2, true>(A, lda, sa, lds, W, sw, M, Npad, K, m0, n0, smem, acc);
+        bs_mainloop<C, BsNoPre, C::BM < 256, true>(A, lda, sa, lds, W, sw, M, Npad, K, m0, n0, smem, acc);
     }
     int wm0, wn0;
     bs_wave_origin<C>(wm0, wn0);
@@ -167,8 +172,7 @@ __global__ void __launch_bounds__(C::NT) k_gemm(const uint8_t *__restrict__ A, i
         constexpr int LPR = S::PC / 8, RPI = 64 / LPR;  // lanes a row, rows a store
         float *tr = (float *)(smem + (threadIdx.x >> 6) * S::SLICE);
         const int rs = lane / LPR, ch = lane % LPR;
-#pragma unroll
-        for (int pass = 0; pass < C::WN / S::PC; pass++) {
+        auto park = [&](int pass) {
             if (pass) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the previous pass's slice reads are done
 #pragma unroll
             for (int i = 0; i < C::TM; i++)
@@ -178,42 +182,76 @@ __global__ void __launch_bounds__(C::NT) k_gemm(const uint8_t *__restrict__ A, i
                     *(float4 *)(tr + (16 * i + c16) * S::LD + 16 * j + 4 * g) = make_float4(v[0], v[1], v[2], v[3]);
                 }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the slice is the wave's own: no block barrier needed
-            const int col = n0 + wn0 + S::PC * pass + 8 * ch;
+        };
+        auto packed = [&](int rr) {
+            const float *t = tr + rr * S::LD + 8 * ch;
+            const float4 a = *(const float4 *)t, b = *(const float4 *)(t + 4);
+            return v4u{f2bf(a.x) | (uint32_t)f2bf(a.y) << 16, f2bf(a.z) | (uint32_t)f2bf(a.w) << 16,
+                       f2bf(b.x) | (uint32_t)f2bf(b.y) << 16, f2bf(b.z) | (uint32_t)f2bf(b.w) << 16};
+        };
+        if constexpr (OUT == 2) {
+            const __amdgpu_buffer_rsrc_t rc = buf_rsrc(Cp, (uint32_t)M * (uint32_t)ldc * 2u);
 #pragma unroll
-            for (int it = 0; it < C::WM / RPI; it++) {
-                const int rr = RPI * it + rs, row = m0 + wm0 + rr;
-                const float *t = tr + rr * S::LD + 8 * ch;
-                const float4 a = *(const float4 *)t, b = *(const float4 *)(t + 4);
-                uint16_t *c = (uint16_t *)Cp + (size_t)row * ldc + col;
-                if (row < M && col + 8 <= N) {
-                    *(v4u_e *)c = v4u_e{f2bf(a.x) | (uint32_t)f2bf(a.y) << 16, f2bf(a.z) | (uint32_t)f2bf(a.w) << 16,
-                                        f2bf(b.x) | (uint32_t)f2bf(b.y) << 16, f2bf(b.z) | (uint32_t)f2bf(b.w) << 16};
-                } else if (row < M) {
-                    for (int e = 0; col + e < N; e++) c[e] = f2bf(t[e]);
+            for (int pass = 0; pass < C::WN / S::PC; pass++) {
+                park(pass);
+                const int col = n0 + wn0 + S::PC * pass + 8 * ch;
+#pragma unroll
+                for (int it = 0; it < C::WM / RPI; it++) {
+                    const int rr = RPI * it + rs;
+                    const v4u o = packed(rr);
+                    if (col < N)
+                        __builtin_amdgcn_raw_buffer_store_b128(
+                            o, rc, (int)(((uint32_t)(m0 + wm0 + rr) * (uint32_t)ldc + (uint32_t)col) * 2u), 0, 0);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int pass = 0; pass < C::WN / S::PC; pass++) {
+                park(pass);
+                const int col = n0 + wn0 + S::PC * pass + 8 * ch;
+#pragma unroll
+                for (int it = 0; it < C::WM / RPI; it++) {
+                    const int rr = RPI * it + rs, row = m0 + wm0 + rr;
+                    const float *t = tr + rr * S::LD + 8 * ch;
+                    uint16_t *c = (uint16_t *)Cp + (size_t)row * ldc + col;
+                    if (row < M && col + 8 <= N) {
+                        *(v4u_e *)c = packed(rr);
+                    } else if (row < M) {
+                        for (int e = 0; col + e < N; e++) c[e] = f2bf(t[e]);
+                    }
                 }
             }
         }
     }
 }
 
-// Tiles by how many there are (us; bf16 output, dense unless said):
-//  - 64 x 64 while one round of two blocks per CU holds them: 128 x 128 -> 64 x 64 at 1 x 1000 x 4736 (M x N x K) 22.5 ->
-//    12.0, 100 x 13461 x 1024 10.9 -> 7.3, 1025 x 1024 x 1024 7.8 -> 6.1 (64 x 128: 16.5, 8.7, 6.6);
+// Tiles by how many there are (us; bf16 output, dense unless said; M x N x K):
+//  - 64 x 64 while one round of two blocks per CU holds them: 128 x 128 -> 64 x 64 at 1 x 1000 x 4736 22.5 -> 12.0,
+//    100 x 13461 x 1024 10.9 -> 7.3, 1025 x 1024 x 1024 7.8 -> 6.1 (64 x 128: 16.5, 8.7, 6.6);
 //  - 64 x 128 likewise: 1025 x 3072 x 1024 9.05 -> 8.7, x 4736 31.9 -> 25.1 (64 x 64: 10.4, 32.2);
-//  - 256 x 256 where they fill one round, or 1.6 and more (2:4-sparse 4322 x 6256 x 4608 116.7 against 121.4): 4100 x
-//    3072 x 1024 19.8 against 21.6 for 128 x 128, 2:4-sparse 8200 x 13456 x 1024 138 against 146;
-//  - 128 x 128 elsewhere: 2050 x 3072 x 1024 18.1 -> 12.6, 1025 x 13461 x 1024 51.1 -> 39.5, 4100 x 5000 x 2048 61.2 ->
-//    55.6 (the tile before was 256 x 256 from 256 of them on).
+//  - 256 x 256 from 1.6 rounds of one block per CU on, and for one round where 128 x 128 would take more than 1.5 rounds
+//    of two per CU: 3584 x 3584 x 1024 21.7 -> 20.4, 4096 x 3840 x 512 14.5 -> 13.2, 2:4-sparse 5000 x 2560 x 1024 21.6
+//    -> 19.6; dense from K = 2048 on also at those 1.5 rounds (3000 x 4096 x 2048 33.0 -> 30.5; x 512 13.4 -> 13.8) and
+//    past the next 1.5 (8200 x 3072 x 3072 92.4 -> 81.2; x 512 23.4 -> 24.6);
+//  - 128 x 128 elsewhere, in 8 waves (LayerMid) where the last round holds at most one block per CU, which then has two
+//    waves per SIMD (4 waves: 8200 x 2048 x 1024 27.5 against 25.9, 8100 x 3000 x 2048 with a full last round 58.8
+//    against 60.5), and for 2:4-sparse weights past the K below (4 waves: 2050 x 3072 x 3072 28.6 against 26.7, x 128
+//    6.4 against 6.6); in 4 waves (GemmMid) where two blocks per CU run to the end: 8 -> 4 waves 2050 x 3072 x 512 8.9
+//    -> 8.5, 1143 x 6768 x 1536 17.5 -> 16.5, 4896 x 840 x 3072 26.2 -> 24.6; not for a bf16 C that is not aligned (1877
+//    x 12690 x 128 15.1 against 16.3).
 typedef BsCfg<64, 64, 2, 2, 3> GemmSml;
-template <class F>
-static void with_gemm_cfg(int M, int N, F f)
+typedef BsCfg<128, 128, 2, 2, 2> GemmMid;
+template <bool SP, class F>
+static void with_gemm_cfg(int M, int N, int K, int out, F f)  // out as k_gemm's OUT
 {
     auto tiles = [&](auto c) { return (long)((M + c.BM - 1) / c.BM) * ((N + c.BN - 1) / c.BN); };
-    const long big = tiles(LayerCfg{});
+    const long big = tiles(LayerCfg{}), last = tiles(LayerMid{}) % 512;
+    const bool deep = !SP && K >= 2048;
     if (tiles(GemmSml{}) <= 512) f(GemmSml{});
     else if (tiles(LayerSml{}) <= 512) f(LayerSml{});
-    else if ((big >= 192 && big <= 256) || big >= 410) f(LayerCfg{});
-    else f(LayerMid{});
+    else if (big >= (deep ? 385 : 410) || (big >= (deep ? 192 : 193) && big <= 256)) f(LayerCfg{});
+    else if ((last > 0 && last < 256) || (SP && K > (out == 1 ? 896 : 128)) || !out) f(LayerMid{});
+    else f(GemmMid{});
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -292,13 +330,19 @@ static int gemm_launch(const char *what, const void *qa, int lda, const float *s
     const uint8_t *A = (const uint8_t *)qa, *W = (const uint8_t *)qw;
     const uint32_t *X = (const uint32_t *)qx;
     hipStream_t st = (hipStream_t)stream;
-    with_gemm_cfg(M, N, [&](auto c_) {
+    // the descriptor's 32-bit offsets must not wrap for the rows of the last tile past M
+    const bool aligned = ((ldc | N) & 7) == 0 && ((uintptr_t)c & 15) == 0 && ((size_t)M + 256) * ldc * 2 < (1ull << 32);
+    const int out = out_kind ? 1 : aligned ? 2 : 0;
+    with_gemm_cfg<SP>(M, N, K, out, [&](auto c_) {
         using T = decltype(c_);
         const dim3 grid((unsigned)(((M + T::BM - 1) / T::BM) * ((N + T::BN - 1) / T::BN)));
-        if (out_kind == 0)
-            hipLaunchKernelGGL((k_gemm<T, 0, SP>), grid, dim3(T::NT), 0, st, A, lda, sa, lds, W, X, sw, c, ldc, M, N, K);
-        else
-            hipLaunchKernelGGL((k_gemm<T, 1, SP>), grid, dim3(T::NT), 0, st, A, lda, sa, lds, W, X, sw, c, ldc, M, N, K);
+        constexpr bool wide = T::TM == 4;  // the tiles with a kernel for an aligned C
+        auto run = [&](auto kern) {
+            hipLaunchKernelGGL(kern, grid, dim3(T::NT), 0, st, A, lda, sa, lds, W, X, sw, c, ldc, M, N, K);
+        };
+        if (out == 1) run(k_gemm<T, 1, SP>);
+        else if (wide && out == 2) run(k_gemm<T, wide ? 2 : 0, SP>);
+        else run(k_gemm<T, std::is_same_v<T, GemmMid> ? 2 : 0, SP>);  // GemmMid: out is never 0
     });
     return xt_check(what);
 }
