@@ -222,8 +222,11 @@ def test_gemm_any_alignment_and_tile(dev, xt, M, N, K, off, pad, sparse):
         assert torch.equal(buf, want)
 
 
+PX_FC1_ROWS = [2048, 2049, 3328, 3329, 12288, 12289]
+
+
 @pytest.mark.parametrize("with_rs", [False, True])
-@pytest.mark.parametrize("rows", [12288, 12289])
+@pytest.mark.parametrize("rows", PX_FC1_ROWS)
 def test_px_fc1_rows_do_not_depend_on_the_tile(dev, xt, rows, with_rs):
     print(f"px fc1: {rows} rows, rs {with_rs}", flush=True)
     L, P, st = xt.lib, xt.ptr, torch.cuda.current_stream().cuda_stream

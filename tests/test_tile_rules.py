@@ -79,7 +79,11 @@ def test_both_sides_of_every_limit(tile):
         for x in limits[:2]:
             assert x in rows and x + 1 in rows, x
     assert _limits(tile, "fc1", 20000) == [1408] and {1408, 1409} <= set(G.RES_ROWS)
-    assert _limits(tile, "px_fc1", 20000) == [12288]
+    wide = (128, 128, 4)
+    for rows, want in ((1, wide), (2048, wide), (2049, BIG), (3328, BIG), (3329, wide), (5184, wide), (5377, BIG),
+                       (6656, BIG), (6657, wide), (10368, wide), (12288, wide), (12289, BIG), (20736, BIG)):
+        assert tile("px_fc1", rows) == want, rows
+    assert {tile("px_fc1", r) for r in G.PX_FC1_ROWS} == {wide, BIG}
     assert [tile("qkv", 1025 * nb) for nb in (1, 2, 3, 5, 6, 7, 8, 16, 32)] == [MID, MID, BIG, BIG, MID, BIG, BIG, BIG, BIG]
     assert [tile("pe", r) for r in (1024, 2048, 2049, 3072)] == [(64, 64, 4), (64, 64, 4), MID, MID]
 

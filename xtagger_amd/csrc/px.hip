@@ -294,15 +294,18 @@ extern "C" int px_k_fc2(const void *m8, const float *ms, int lds, const void *w,
     return xt_px_fc2(m8, ms, lds, w, ws, bias, x, rows, 1, stream);
 }
 
-// k_px_fc1's tiles: 128 x 128 (4 waves of 32 x 128, two blocks per CU) up to 12288 rows: one block's GELU and packing
-// runs beside the other's main loop, and the last round wastes less (48.0 -> 41.4 us at 5184 rows, 85.2 -> 77.0 at
-// 10368); with more rounds 256 x 256 is as good or better (111 against 114 at 15552, 290 against 292 at 41472), and so
-// it is beside an engine's other lane, which covers them too (a batch of 6 images 23740 -> 23540 us, of 4 the same).
+// k_px_fc1's tiles: 128 x 128 (4 waves of 32 x 128, two blocks per CU) up to 12288 rows, where the last round of
+// 256 x 256 would fill at most 0.6 of the CUs: one block's GELU and packing runs beside the other's main loop, and the
+// last round wastes less (us, 256 x 256 -> 128 x 128: 20.5 -> 12.5 at 1024 rows, 43.1 -> 38.0 at 5184, 84.1 -> 72.3 at
+// 10368). With a fuller last round 256 x 256 is 3 to 6% faster (23.3 against 24.8 at 3200, 43.5 against 46.3 at 6272,
+// 66.1 against 70.5 at 10112), with more rounds as good (111 against 114 at 15552, 290 against 292 at 41472), and so it
+// is beside an engine's other lane, which takes the CUs that a round leaves (a batch of 6 images 23740 -> 23540 us).
 typedef BsCfg<128, 128, 4, 1, 2> PxFc1Mid;
 template <class F>
 static void with_px_fc1_cfg(int rows, int lanes, F f)
 {
-    if (lanes == 1 && rows <= 12288) f(PxFc1Mid{});
+    const unsigned last = layer_grid<LayerCfg>(rows, PX_HID) % 256;
+    if (lanes == 1 && rows <= 12288 && last > 0 && last <= 152) f(PxFc1Mid{});
     else f(LayerCfg{});
 }
 
